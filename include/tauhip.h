@@ -37,7 +37,7 @@
 extern "C" {
 #endif
 
-#define TF_ABI_VERSION 12
+#define TF_ABI_VERSION 13
 
 #define TF_KIND_SOLVER 0
 #define TF_KIND_MULTIPHASE 1
@@ -95,6 +95,19 @@ typedef struct tf_tile {
  * values (zeros).  The sweep reads the field in 16-byte quads that start up
  * to 3 voxels before z = 0. */
 #define TF_FIELD_SLACK_BYTES 16
+
+/* Layout of the resident sweep (tf_sweep_resident): `elems` consecutive
+ * voxels of a row per lane (the row lies along z, or along y when lane_y),
+ * patches of px x py rows per wave, wx x wy waves per workgroup (waves =
+ * wx * wy), `tiles` workgroups, and the bytes of mailbox they exchange faces
+ * through. */
+typedef struct tf_resident {
+    int elems, px, py, waves, wy, lane_y, tiles, reserved;
+    long long mail_bytes;
+} tf_resident;
+
+/* status of tf_sweep_resident: the device cannot hold the workgroups at once */
+#define TF_NOT_RESIDENT (-2)
 
 /* ABI version of the loaded library (TF_ABI_VERSION). No reference
  * counterpart: lets the Python loader refuse a stale build. */
@@ -460,6 +473,34 @@ int tf_spans_x(const uint8_t* mask, int X, int Y, int Z);
  * calibrates the HBM traffic counters and gives the device's copy rate
  * against which the sweep's measured traffic is read.                    */
 int tf_hbm_copy(const void* src, void* dst, long long bytes, void* stream);
+
+/* Resident sweep: a volume that fits into the registers of the device at
+ * once, any number of half-sweeps in one launch (same iterates as tf_sweep).
+ *
+ * tf_resident_plan chooses the layout for `kind` (TF_KIND_SOLVER,
+ * TF_KIND_ANISOTROPIC or TF_KIND_ELECTRODE, optionally with
+ * TF_SWEEP_PERIODIC_YZ) on a device of compute_units CUs: 1 and *plan if the
+ * volume fits, 0 if it does not.  Host only.
+ *
+ * tf_sweep_resident runs n_half half-sweeps from src into dst (distinct, both
+ * with their ghosts set; only the interior of dst is written).
+ *   codes     the sweep codes, as tf_sweep
+ *   table     as hm_lut of tf_sweep (null for TF_KIND_SOLVER)
+ *   mail      plan->mail_bytes of 8-byte aligned device memory, zero before
+ *             the first launch, used by one launch at a time
+ *   tag       counts the half-sweeps of all launches on this mailbox: at
+ *             least 1, and the next launch's at least tag + n_half + 1
+ *   status    one device int, 0: the workgroups wait for each other's faces,
+ *             and if a wait ends after `spin` polls (0: a default of some
+ *             50 ms) the launch stores launch_id (> 0) there and dst is void;
+ *             a launch that finds it nonzero writes nothing.
+ * TF_NOT_RESIDENT if the device cannot hold the workgroups at once (nothing
+ * is launched). */
+int tf_resident_plan(int kind, int B, int X, int Y, int Z, int compute_units, tf_resident* plan);
+int tf_sweep_resident(const float* src, float* dst, const uint8_t* codes, const float* table,
+                      int kind, int B, int X, int Y, int Z, float omega, int first_colour,
+                      int n_half, const tf_resident* plan, void* mail, long long mail_bytes,
+                      uint32_t tag, int* status, int launch_id, int spin, void* stream);
 
 #ifdef __cplusplus
 }

@@ -11,7 +11,7 @@ import threading
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libtauhip.so")
-ABI_VERSION = 12
+ABI_VERSION = 13
 
 KIND_SOLVER = 0
 KIND_MULTIPHASE = 1
@@ -42,6 +42,15 @@ class Tile(ctypes.Structure):
     _fields_ = [("waves", ctypes.c_int), ("rows_per_wave", ctypes.c_int), ("tx", ctypes.c_int)]
 
 
+class Resident(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int) for n in ("elems", "px", "py", "waves", "wy", "lane_y", "tiles", "reserved")] + \
+        [("mail_bytes", ctypes.c_longlong)]
+
+
+# status of tf_sweep_resident: the device cannot hold the workgroups at once
+NOT_RESIDENT = -2
+
+
 # name -> (restype, argtypes); the exported surface of include/tauhip.h
 SIGNATURES = {
     "tf_abi_version": (_c_int, []),
@@ -59,6 +68,10 @@ SIGNATURES = {
     "tf_multiphase_face_codes": (_c_int, [_vp, _vp, _c_int, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _vp]),
     "tf_sweep": (_c_int, [_vp, _vp, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                           _c_float, _c_int, _c_int, ctypes.POINTER(Tile), _vp]),
+    "tf_resident_plan": (_c_int, [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, ctypes.POINTER(Resident)]),
+    "tf_sweep_resident": (_c_int, [_vp, _vp, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int,
+                                   _c_int, ctypes.POINTER(Resident), _vp, ctypes.c_longlong, ctypes.c_uint32, _vp,
+                                   _c_int, _c_int, _vp]),
     "tf_sweep_half_inplace": (_c_int, [_vp, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_int,
                                        _c_int, _c_float, _c_int, _vp]),
     "tf_layer_sums": (_c_int, [_vp, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,

@@ -1,0 +1,6 @@
+// Resident sweep kernels of the anisotropic kind: every compiled shape of k_resident.
+#include "tauhip_resident.h"
+
+int resident_dispatch_anisotropic(const tf_resident& p, const ResidentArgs& a, hipStream_t st) {
+    return dispatch_resident<TF_KIND_ANISOTROPIC, false>(p, a, st);
+}

@@ -10,7 +10,7 @@
 // Layout and conventions are documented in include/tauhip.h.  The sweep
 // kernels live in tauhip_sweep.h and are instantiated in sweep_<kind>.hip.
 
-#include "tauhip_sweep.h"
+#include "tauhip_resident.h"
 
 #include <mutex>
 
@@ -589,6 +589,131 @@ extern "C" int tf_sweep_launch_config(int kind, int n_classes, int B, int X, int
     out->tx = a.TX;
     if (n_tiles) *n_tiles = a.total;
     return 0;
+}
+
+// ---------------------------------------------------------------------------
+// resident sweep: layout and launch
+// ---------------------------------------------------------------------------
+struct ResidentShapeDesc {
+    int elems, px, py, waves;
+    size_t (*lds_floats)(int wy);  // of the kind with the largest table
+};
+static const ResidentShapeDesc kResidentShapes[] = {
+#define F(P, PX, PY, NW) {P, PX, PY, NW, ResidentShape<TF_KIND_ANISOTROPIC, P, PX, PY, NW>::lds_floats},
+    TF_RESIDENT_SHAPES(F)
+#undef F
+};
+
+// Geometry of one shape with wx x wy waves; false if the volume does not fit
+// it.  A wave asks for at most one face per axis from another workgroup
+// (k_resident's poll): a tile has at least two waves along an axis that it
+// does not span, and with wrapped rows the last tile too.
+static bool resident_geometry(const ResidentShapeDesc& s, int wy, int B, int X, int lane_n, int row_n,
+                              bool periodic, long long* ntx, long long* nty) {
+    if (wy < 1 || s.waves % wy) return false;
+    const int wx = s.waves / wy;
+    if (lane_n > 64 * s.elems) return false;
+    if (periodic && (lane_n % s.elems || row_n % s.py)) return false;
+    const long long ngx = (X + s.px - 1) / s.px, ngy = (row_n + s.py - 1) / s.py;
+    *ntx = (ngx + wx - 1) / wx;
+    *nty = (ngy + wy - 1) / wy;
+    if (*ntx > 1 && wx < 2) return false;
+    if (*nty > 1 && wy < 2) return false;
+    if (periodic && *nty > 1 && ngy % wy == 1) return false;
+    return *ntx * *nty * B <= (1 << 20);
+}
+
+static long long resident_mail_bytes(const ResidentShapeDesc& s, int wy, long long tiles) {
+    const long long rows = 2LL * (wy * s.py + s.waves / wy * s.px);
+    return tiles * 2 * rows * (s.elems / 2) * 64 * 8;
+}
+
+static int resident_kind(int& kind, int& periodic, int Y, int Z) {
+    if (int rc = split_sweep_kind(kind, periodic, Y, Z)) return rc;
+    if (!own_code_kind(kind)) return fail(-1, "no resident sweep of kind %d", kind);
+    return 0;
+}
+
+extern "C" int tf_resident_plan(int kind, int B, int X, int Y, int Z, int compute_units, tf_resident* plan) {
+    if (!plan) return fail(-1, "null pointer argument");
+    if (int rc = check_dims(B, X, Y, Z)) return rc;
+    int periodic = 0;
+    if (int rc = resident_kind(kind, periodic, Y, Z)) return rc;
+    // rows along z; a 2-D image's pixels lie along y
+    const int lane_y = Z == 1 && Y > 1;
+    const int lane_n = lane_y ? Y : Z, row_n = lane_y ? 1 : Y;
+    long long best = -1, best_mail = 0;
+    for (const ResidentShapeDesc& s : kResidentShapes) {
+        // the fewest voxels per lane that cover a row
+        if (lane_n > 64 * s.elems || (s.elems > 2 && lane_n <= 32 * s.elems)) continue;
+        for (int wy = 1; wy <= s.waves; ++wy) {
+            long long ntx, nty;
+            if (!resident_geometry(s, wy, B, X, lane_n, row_n, periodic != 0, &ntx, &nty)) continue;
+            const long long tiles = ntx * nty * B;
+            if ((tiles + 7) / 8 * 8 > compute_units) continue;
+            if (s.lds_floats(wy) * sizeof(float) > 160 * 1024) continue;
+            // the least work per compute unit, then the least mail
+            const long long work = (long long)s.waves * s.px * s.py * s.elems;
+            const long long mail = resident_mail_bytes(s, wy, tiles);
+            if (best >= 0 && (work > best || (work == best && mail >= best_mail))) continue;
+            best = work;
+            best_mail = mail;
+            *plan = tf_resident{s.elems, s.px, s.py, s.waves, wy, lane_y, (int)tiles, 0, mail};
+        }
+    }
+    return best >= 0 ? 1 : 0;
+}
+
+extern "C" int tf_sweep_resident(const float* src, float* dst, const uint8_t* codes, const float* table,
+                                 int kind, int B, int X, int Y, int Z, float omega, int first_colour,
+                                 int n_half, const tf_resident* plan, void* mail, long long mail_bytes,
+                                 uint32_t tag, int* status, int launch_id, int spin, void* stream) {
+    if (int rc = check_dims(B, X, Y, Z)) return rc;
+    int periodic = 0;
+    if (int rc = resident_kind(kind, periodic, Y, Z)) return rc;
+    if (!src || !dst || !codes || !plan || !mail || !status || (kind != TF_KIND_SOLVER && !table))
+        return fail(-1, "null pointer argument");
+    if (src == dst) return fail(-1, "tf_sweep_resident needs distinct src and dst buffers");
+    if (first_colour != 0 && first_colour != 1) return fail(-1, "first_colour must be 0 or 1");
+    if (n_half < 1 || n_half > (1 << 20)) return fail(-1, "n_half=%d out of range", n_half);
+    if (launch_id < 1 || spin < 0) return fail(-1, "invalid launch_id %d or spin %d", launch_id, spin);
+    if (tag < 1 || (uint64_t)tag + n_half + 1 > 0xffffffffu) return fail(-1, "tag %u out of range", tag);
+    const ResidentShapeDesc s{plan->elems, plan->px, plan->py, plan->waves, nullptr};
+    if (s.elems < 2 || s.px < 1 || s.py < 1 || s.waves < 1) return fail(-1, "invalid resident layout");
+    const bool lane_y = plan->lane_y != 0;
+    if (lane_y && Z != 1) return fail(-1, "rows along y need Z = 1");
+    ResidentArgs a = {};
+    a.v = make_vol(X, Y, Z);
+    a.lane_n = lane_y ? Y : Z;
+    a.row_n = lane_y ? 1 : Y;
+    a.sL = lane_y ? a.v.sY : 1;
+    a.sR = lane_y ? 1 : a.v.sY;
+    a.cX = (Y + 2) * sweep_code_row(Z);
+    a.cL = lane_y ? sweep_code_row(Z) : 1;
+    a.cR = lane_y ? 1 : sweep_code_row(Z);
+    long long ntx, nty;
+    if (!resident_geometry(s, plan->wy, B, X, a.lane_n, a.row_n, periodic != 0, &ntx, &nty))
+        return fail(-1, "the resident layout does not fit the volume");
+    a.nTx = (int)ntx;
+    a.nTy = (int)nty;
+    a.total = (int)(ntx * nty * B);
+    const long long need = resident_mail_bytes(s, plan->wy, a.total);
+    if (mail_bytes < need || ((uintptr_t)mail & 7))
+        return fail(-1, "a mailbox of %lld 8-byte aligned bytes is needed (got %lld)", need, mail_bytes);
+    a.src = src; a.dst = dst; a.codes = codes; a.table = table;
+    a.w = omega;
+    a.colour0 = first_colour;
+    a.n_half = n_half;
+    a.WY = plan->wy;
+    a.mail = static_cast<unsigned long long*>(mail);
+    a.tag0 = tag;
+    a.status = status;
+    a.launch_id = launch_id;
+    a.spin = spin > 0 ? spin : kResidentSpin;
+    const hipStream_t st = (hipStream_t)stream;
+    if (kind == TF_KIND_ANISOTROPIC) return resident_dispatch_anisotropic(*plan, a, st);
+    if (kind == TF_KIND_ELECTRODE) return resident_dispatch_electrode(*plan, a, periodic, st);
+    return periodic ? resident_dispatch_periodic(*plan, a, st) : resident_dispatch_solver(*plan, a, st);
 }
 
 // ---------------------------------------------------------------------------

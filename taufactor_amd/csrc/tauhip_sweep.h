@@ -118,6 +118,19 @@ __device__ __forceinline__ float div_by_count(float s, float r, float d, int cod
     return q;
 }
 
+// (1/f, f) of a prefactor table entry for the reciprocal division of the
+// anisotropic and electrode kinds; inf (an inert voxel) is the pair (0, 0).
+// q = s (1/f) and one residual correction is s / f correctly rounded for a
+// correctly rounded 1/f, f in [2^-20, 2^20] and |s| >= 2^-100 (Markstein's
+// correction step: the residual is exact); `odd` reports a prefactor outside
+// that range (a NaN among them), for which a launch divides throughout.
+__device__ __forceinline__ void prefactor_pair(float f, float& r, float& g, bool& odd) {
+    const bool inert = f == __builtin_inff();
+    odd = !inert && !(f >= 0x1p-20f && f <= 0x1p20f);
+    r = inert ? 0.0f : 1.0f / f;
+    g = inert ? 0.0f : f;
+}
+
 // table of (1/d, d) per Solver code; code 0 means factor = inf
 static __constant__ float c_rcp[9] = {0.0f, 1.0f, 0.5f, 1.0f / 3.0f, 0.25f,
                                0.2f, 1.0f / 6.0f, 1.0f / 7.0f, 0.125f};

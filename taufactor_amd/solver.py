@@ -106,14 +106,16 @@ class SORSolver(ABC):
             # per-layer float64 sums, flux (B x (X-1), or B x X for the
             # electrode kind) then concentration (B x X), in one buffer so
             # that a check copies them to the host in one transfer
+            # (and, last, the status word of the resident sweeps)
             B, X = self.batch_size, self.Nx
-            self._sums = torch.zeros(2 * B * X, dtype=torch.float64, device=self.device)
-            self._sums_host = torch.empty(2 * B * X, dtype=torch.float64, pin_memory=True)
+            self._sums = torch.zeros(2 * B * X + 1, dtype=torch.float64, device=self.device)
+            self._sums_host = torch.empty(2 * B * X + 1, dtype=torch.float64, pin_memory=True)
             # per-chunk partial sums of tf_layer_sums_ws
             ws = self._lib.tf_layer_sums_workspace_bytes(B, X, self.Ny, self.Nz)
             if ws < 0:
                 _lib.check(int(ws), "tf_layer_sums_workspace_bytes")
             self._sums_ws = torch.empty(max(ws // 8, 1), dtype=torch.float64, device=self.device)
+        self._resident = None  # _ResidentSweep, False once it does not apply
         self._sums_ready = None  # event: sums enqueued, not yet read
         self._ahead = 0  # half-sweeps already launched for the next block
 
@@ -145,8 +147,10 @@ class SORSolver(ABC):
         host image: the initial field the set-up wrote is copied back (the
         codes and tables the set-up built do not change during a solve)."""
         with torch.cuda.device(self.device):
-            for f in self._fields + ([self._spare] if self._spare is not None else []):
+            for f in self._all_fields():
                 self._copy_field(self._field_init, f)
+            if self._resident:
+                self._resident.forget()
         self._cur = 0
         self._ahead = 0
         self._checked = None
@@ -169,9 +173,15 @@ class SORSolver(ABC):
         """Dirichlet in x and no-flux in y and z: held by the ghost layers."""
 
     # ---------------- device state ----------------
+    def _all_fields(self):
+        """Every field buffer a launch may write."""
+        extra = [self._spare, self._resident.third if self._resident else None]
+        return self._fields + [f for f in extra if f is not None]
+
     @property
     def field(self) -> torch.Tensor:
         """Current padded field [B, Nx+2, Ny+2, Nz+2] (float32, on device)."""
+        self._settle()
         return self._fields[self._cur]
 
     @field.setter
@@ -185,7 +195,8 @@ class SORSolver(ABC):
         if self._zero_yz_ghosts and value.dim() == 4 and (
                 torch.any(value[:, :, [0, -1], :] != 0) or torch.any(value[:, :, :, [0, -1]] != 0)):
             raise ValueError("the y/z ghost layers of the field must hold 0 (closed boundaries)")
-        for f in self._fields + ([self._spare] if self._spare is not None else []):
+        self._settle()
+        for f in self._all_fields():
             f.copy_(value)
 
     @property
@@ -297,12 +308,15 @@ class SORSolver(ABC):
         _lib.check(st, "tf_sweep")
         self._cur = 1 - self._cur
 
-    def _advance(self, n_half: int) -> None:
+    def _advance(self, n_half: int, resident: bool = True) -> None:
         """Run n_half reference iterations (half-sweeps) on the device; the
-        first self._ahead of them were launched ahead of the last check."""
+        first self._ahead of them were launched ahead of the last check.
+        resident False: with streaming launches in any case."""
         done, self._ahead = self._ahead, 0
         it = self.iter + done
         n_half -= done
+        if n_half > 0 and resident and self._resident_sweep() and self._resident.launch(self, n_half, it):
+            return
         per, tile, codes, hm = self._sweep_args()
         # timing (bench.py): HIP events on the launch stream around the
         # launches that fuse the full `per` half-sweeps (a shorter last
@@ -345,6 +359,11 @@ class SORSolver(ABC):
         room = self._ahead_room(n_next)
         if room <= 0:
             return
+        if self._resident_sweep():
+            n = min(room, self.RESIDENT_AHEAD)
+            if self._resident.launch(self, n, self.iter):
+                self._ahead = n
+                return
         per, tile, codes, hm = self._sweep_args()
         launches = 1
         if self._spare is not None:
@@ -364,6 +383,8 @@ class SORSolver(ABC):
 
     def _drop_ahead(self) -> None:
         if self._ahead:
+            if self._resident:
+                self._resident.drop_from(self.iter)
             if self._checked is not None:
                 fields, cur = self._checked
                 pool = self._fields + [self._spare]
@@ -374,14 +395,54 @@ class SORSolver(ABC):
             self._ahead = 0
         self._checked = None
 
+    # iterations launched ahead of a check decision by the resident sweep
+    RESIDENT_AHEAD = 40
+
+    def _resident_sweep(self) -> bool:
+        """Do the launches of this solver run as resident sweeps?  Where the
+        kind has one and the volume fits the device (tf_resident_plan),
+        unless the launch configuration was set by hand."""
+        if self.half_sweeps_per_pass is not None or self.tile is not None:
+            return False
+        if self._resident is None:
+            self._resident = _ResidentSweep.make(self) or False
+        return bool(self._resident)
+
+    def _settle(self) -> None:
+        """Make sure that the resident launches since the last check ran to
+        their end (waits for them); repeat them otherwise."""
+        if self._resident and self._resident.log:
+            status = int(self._resident.status.item())
+            if status:
+                self._recover(status)
+            elif self._resident:
+                self._resident.log.clear()
+
+    def _recover(self, status: int) -> None:
+        """A resident launch did not get all its workgroups onto the device
+        in time (status, its number) and the launches after it wrote nothing:
+        go back to what it read and repeat with the streaming sweep, as
+        will this solver's later launches."""
+        r, self._resident = self._resident, False
+        lost = next((e for e in r.log if e[0] >= status), None)
+        if lost is None:
+            return  # only launches that were dropped since
+        _, src, it = lost
+        other = next(f for f in self._fields + ([r.third] if r.third is not None else []) if f is not src)
+        self._fields, self._cur = [src, other], 0
+        self._ahead, self._checked, self._sums_ready = 0, None, None
+        end, self.iter = self.iter, it
+        self._advance(end - it)
+        self.iter = end
+
     def _enqueue_layer_sums(self) -> None:
         """Layer sums of the current field and their copy to pinned host
         memory, enqueued on the launch stream; _layer_sums waits for them."""
         B, X, Y, Z = self.batch_size, self.Nx, self.Ny, self.Nz
         flux = self._sums[:B * X]
-        conc = self._sums[B * X:]
+        conc = self._sums[B * X:2 * B * X]
         st = self._lib.tf_layer_sums_ws(
-            _lib.ptr(self.field), _lib.ptr(self._codes),
+            _lib.ptr(self._fields[self._cur]), _lib.ptr(self._codes),
             _lib.ptr(self._hm_lut) if self._hm_lut is not None else None,
             self._n_classes, self.kind, B, X, Y, Z,
             _lib.ptr(flux), _lib.ptr(conc), _lib.ptr(self._sums_ws), self._sums_ws.numel() * 8,
@@ -398,12 +459,18 @@ class SORSolver(ABC):
             self._enqueue_layer_sums()
         self._sums_ready.synchronize()
         self._sums_ready = None
+        if self._resident and self._resident.log:
+            status = int(self._sums_host.numpy()[-1:].view(np.int32)[0])
+            if status:
+                self._recover(status)
+                return self._layer_sums()
+            self._resident.drop_until(self.iter)
         B, X = self.batch_size, self.Nx
         h = self._sums_host.numpy()
         # X - 1 internal faces; the electrode fluxes also have the left face
         width = X if self.kind == _lib.KIND_ELECTRODE else X - 1
         flux = h[:B * width].reshape(B, width).copy()
-        conc = h[B * X:].reshape(B, X).copy()
+        conc = h[B * X:2 * B * X].reshape(B, X).copy()
         return flux, conc
 
     # ---------------- convergence ----------------
@@ -520,6 +587,74 @@ class SORSolver(ABC):
             print(f"GPU-RAM currently {torch.cuda.memory_allocated(device=self.device) / 1e6:.2f} MB "
                   f"(max allocated {torch.cuda.max_memory_allocated(device=self.device) / 1e6:.2f} MB; "
                   f"{torch.cuda.max_memory_reserved(device=self.device) / 1e6:.2f} MB reserved)")
+
+
+class _ResidentSweep:
+    """The resident sweep of one solver (tf_sweep_resident): its layout,
+    mailbox and the launches not yet known to have run to their end."""
+
+    @classmethod
+    def make(cls, s):
+        kind = s.kind | s._sweep_flags
+        if s.kind not in (_lib.KIND_SOLVER, _lib.KIND_ANISOTROPIC, _lib.KIND_ELECTRODE):
+            return None
+        plan = _lib.Resident()
+        cus = torch.cuda.get_device_properties(s.device).multi_processor_count
+        r = s._lib.tf_resident_plan(kind, s.batch_size, s.Nx, s.Ny, s.Nz, cus, ctypes.byref(plan))
+        if r < 0:
+            _lib.check(r, "tf_resident_plan")
+        return cls(s, kind, plan) if r else None
+
+    def __init__(self, s, kind, plan):
+        self.kind, self.plan = kind, plan
+        self.mail = torch.zeros(plan.mail_bytes // 8, dtype=torch.int64, device=s.device)
+        self.status = s._sums[-1:].view(torch.int32)[:1]
+        self.third = None  # see _PeriodicYZ._advance
+        self.spin = 0
+        self.tag, self.count = 1, 0
+        self.log = []  # (number, field read, first iteration) of each launch
+
+    def launch(self, s, n: int, it: int) -> bool:
+        """n half-sweeps from iteration it; False if the device does not hold
+        the workgroups (the solver streams from then on)."""
+        if self.tag + n + 1 >= 2 ** 32:
+            self.mail.zero_()
+            self.tag = 1
+        src, dst = s._fields[s._cur], s._fields[1 - s._cur]
+        self.count += 1
+        _, codes, table, _ = s._sweep_pointers()
+        ev = s._launch_events
+        if ev is not None:
+            t0, t1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            t0.record()
+        st = s._lib.tf_sweep_resident(_lib.ptr(src), _lib.ptr(dst), codes, table, self.kind, s.batch_size, s.Nx,
+                                      s.Ny, s.Nz, s._w32, it & 1, n, self.plan, _lib.ptr(self.mail),
+                                      self.plan.mail_bytes, self.tag, _lib.ptr(self.status), self.count, self.spin,
+                                      s._stream())
+        if st == _lib.NOT_RESIDENT and not self.log:
+            s._resident = False
+            return False
+        _lib.check(st, "tf_sweep_resident")
+        if ev is not None:
+            t1.record()
+            ev.append((t0, t1, 1))
+        self.tag += n + 1
+        self.log.append((self.count, src, it))
+        s._cur = 1 - s._cur
+        return True
+
+    def drop_from(self, it: int) -> None:
+        """Forget the launches from iteration it on."""
+        self.log = [e for e in self.log if e[2] < it]
+
+    def drop_until(self, it: int) -> None:
+        """The launches before iteration it ran to their end."""
+        self.log = [e for e in self.log if e[2] >= it]
+
+    def forget(self) -> None:
+        """The fields were set anew: no launch so far matters."""
+        self.log.clear()
+        self.status.zero_()
 
 
 class ThroughTransportSolver(SORSolver):
@@ -1203,6 +1338,19 @@ class _PeriodicYZ:
         # half-sweep follows a ghost wrap of the field it reads
         return n_next - 1 if self._fused_periodic else 0
 
+    def _last_half_sweep(self) -> None:
+        """The half-sweep before a ghost copy, as a streaming launch.  After a
+        resident launch it writes a third buffer: the field that launch read
+        is kept until the launch is known to have run to its end."""
+        r = self._resident
+        if r and r.log:
+            if r.third is None:
+                r.third = _lib.slack_buffer(tuple(self._field_init.shape), torch.float32, self.device)
+                self._copy_field(self._field_init, r.third)
+            k = 1 - self._cur
+            self._fields[k], r.third = r.third, self._fields[k]
+        SORSolver._advance(self, 1, resident=False)
+
     def _advance(self, n_half: int) -> None:
         if self._fused_periodic:
             it = self.iter
@@ -1210,11 +1358,11 @@ class _PeriodicYZ:
                 if n_half > 1:
                     SORSolver._advance(self, n_half - 1)
                     self.iter = it + n_half - 1  # colour of the last iteration
-                src = self.field
-                SORSolver._advance(self, 1)
+                src = self._fields[self._cur]
+                self._last_half_sweep()
             finally:
                 self.iter = it
-            st = self._lib.tf_wrap_ghosts_from(_lib.ptr(src), _lib.ptr(self.field), self.batch_size,
+            st = self._lib.tf_wrap_ghosts_from(_lib.ptr(src), _lib.ptr(self._fields[self._cur]), self.batch_size,
                                                self.Nx, self.Ny, self.Nz, self._stream())
             _lib.check(st, "tf_wrap_ghosts_from")
             return

@@ -120,3 +120,32 @@ def test_sweep_code_layout_size():
         assert row % 4 == 0 and row >= Z + 5
         assert lib.tf_sweep_codes_bytes(X, Y, Z) == (X + 2) * (Y + 2) * row
     assert lib.tf_sweep_codes_bytes(0, 1, 1) < 0
+
+
+def test_resident_plan():
+    """Layouts on 256 compute units: one workgroup per unit at most, rows
+    covered by the lanes, none for volumes the registers do not hold or kinds
+    without the resident sweep."""
+    lib = _lib.load()
+    p = _lib.Resident()
+
+    def plan(kind, B, X, Y, Z, cus=256):
+        return lib.tf_resident_plan(kind, B, X, Y, Z, cus, ctypes.byref(p))
+
+    for kind, B, X, Y, Z in [(0, 1, 32, 32, 32), (0, 1, 100, 100, 100), (3, 1, 160, 241, 97), (4, 2, 60, 60, 60),
+                             (0, 1, 203, 157, 181), (0, 1, 611, 803, 1), (_lib.SWEEP_PERIODIC_YZ, 1, 64, 64, 64)]:
+        assert plan(kind, B, X, Y, Z) == 1
+        lanes, rows = (Y, 1) if p.lane_y else (Z, Y)
+        assert p.lane_y == (Z == 1) and 64 * p.elems >= lanes and p.waves % p.wy == 0
+        wx = p.waves // p.wy
+        nx, ny = -(-X // (p.px * wx)), -(-rows // (p.py * p.wy))
+        assert p.tiles == nx * ny * B <= 256 and (wx > 1 or nx == 1) and (p.wy > 1 or ny == 1)
+        assert p.mail_bytes == p.tiles * 4 * (p.wy * p.py + wx * p.px) * (p.elems // 2) * 64 * 8
+    assert plan(0, 1, 512, 512, 512) == 0 and plan(0, 1, 100, 100, 100, cus=16) == 0
+    assert plan(0, 1, 8, 8, 2100) == 0  # longer than 64 lanes of 32 voxels
+    assert plan(_lib.SWEEP_PERIODIC_YZ, 1, 20, 20, 130) == 0  # a wrapped row must end with its lane
+    assert plan(_lib.KIND_MULTIPHASE, 1, 8, 8, 8) < 0 and plan(0, 0, 8, 8, 8) < 0
+    assert lib.tf_sweep_resident(1, 1, 1, None, 0, 1, 4, 4, 4, 1.5, 0, 2, p, 1, 8, 1, 1, 1, 0, None) < 0
+    assert plan(0, 1, 40, 40, 40) == 1
+    st = lib.tf_sweep_resident(4, 8, 1, None, 0, 1, 40, 40, 40, 1.5, 0, 2, p, 8, p.mail_bytes - 8, 1, 1, 1, 0, None)
+    assert st < 0 and b"mailbox" in lib.tf_last_error()

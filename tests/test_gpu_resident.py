@@ -1,0 +1,120 @@
+"""GPU: the resident sweep (a volume kept in registers, faces exchanged
+through a mailbox) against the oracle, value for value, at the edges of its
+layout: rows shorter and longer than a wave's lanes, odd sizes, partly filled
+patches and tiles, 2-D images, batches, every kind that has it, and a launch
+whose waits run out."""
+import numpy as np
+import pytest
+import torch
+
+import taufactor_amd as tau
+from oracle.restate import (OracleAnisotropicSolver, OracleElectrodeSolver, OraclePeriodicElectrodeSolver,
+                            OraclePeriodicSolver, OracleSolver)
+
+pytestmark = pytest.mark.gpu
+
+
+def _binary(shape, seed, p=0.65):
+    return (np.random.default_rng(seed).random(shape) < p).astype(np.uint8)
+
+
+def _same(s, o, n):
+    """s after n iterations (resident, two blocks) holds o's field."""
+    s.solve(iter_limit=n, verbose=False, conv_crit=0.0)
+    assert s._resident, "the resident sweep did not run"
+    assert np.array_equal(s.field.cpu().numpy(), o.run(n).field.numpy())
+
+
+# one voxel; rows of 1, 2, 63..65 pairs; rows of 4, 8, 16 and 32 voxels per
+# lane; last patch and last tile partly filled in x and y
+@pytest.mark.parametrize("shape", [(1, 1, 1), (2, 1, 2), (5, 7, 9), (9, 6, 127), (4, 5, 128), (6, 9, 129),
+                                   (7, 10, 255), (3, 4, 257), (17, 33, 30), (66, 5, 3), (5, 9, 600), (2, 3, 1100)])
+def test_solver_shapes(shape):
+    img = _binary(shape, sum(shape))
+    # (a check of a single layer has no fluxes to compare)
+    _same(tau.Solver(img), OracleSolver(img), 109 if shape[0] > 1 else 57)
+
+
+# one volume per compiled shape that the small ones above do not take: (voxels
+# per lane and row, patch, waves) of the plan
+@pytest.mark.parametrize("shape,plan", [
+    ((100, 60, 9), (2, 1, 2, 16)), ((120, 72, 9), (2, 2, 2, 16)), ((130, 130, 9), (2, 2, 4, 16)),
+    ((230, 138, 9), (2, 4, 4, 16)), ((330, 198, 9), (2, 6, 8, 8)), ((100, 60, 140), (4, 1, 2, 16)),
+    ((120, 72, 140), (4, 2, 2, 16)), ((130, 130, 140), (4, 2, 3, 16)), ((215, 129, 140), (4, 2, 4, 16)),
+    ((230, 138, 140), (4, 4, 5, 8)), ((270, 162, 140), (4, 4, 6, 8)), ((100, 60, 260), (8, 1, 2, 16)),
+    ((150, 90, 260), (8, 2, 2, 16)), ((120, 72, 260), (8, 2, 3, 8)), ((130, 130, 260), (8, 3, 4, 8)),
+    ((100, 60, 520), (16, 2, 2, 8))])
+def test_every_patch(shape, plan):
+    img = _binary(shape, 5)
+    s = tau.Solver(img)
+    assert s._resident_sweep()
+    p = s._resident.plan
+    assert (p.elems, p.px, p.py, p.waves) == plan
+    _same(s, OracleSolver(img), 7)
+
+
+@pytest.mark.parametrize("shape", [(1, 2), (33, 40), (16, 129), (40, 300), (9, 515), (35, 1030)])
+def test_images(shape):
+    img = _binary(shape, shape[0], p=0.8)
+    s = tau.Solver(img)
+    assert s._resident_sweep() and s._resident.plan.lane_y
+    _same(s, OracleSolver(img), 109 if shape[0] > 1 else 57)
+
+
+def test_batch():
+    img = np.stack([_binary((18, 21, 23), i) for i in range(3)])
+    _same(tau.Solver(img), OracleSolver(img), 109)
+
+
+@pytest.mark.parametrize("shape", [(12, 2, 2), (9, 10, 12), (8, 34, 128), (20, 18, 132)])
+def test_periodic(shape):
+    """Rows and lanes wrap round, inside a workgroup and across; the ghosts
+    end as the reference's."""
+    img = _binary(shape, 3)
+    _same(tau.PeriodicSolver(img), OraclePeriodicSolver(img), 109)
+
+
+@pytest.mark.parametrize("shape", [(9, 11, 13), (14, 40), (6, 9, 131)])
+def test_anisotropic(shape):
+    img = _binary(shape, 4)
+    _same(tau.AnisotropicSolver(img, (1.0, 1.3, 2.0)), OracleAnisotropicSolver(img, (1.0, 1.3, 2.0)), 109)
+
+
+@pytest.mark.parametrize("periodic", [False, True])
+def test_electrode(periodic):
+    img = np.random.default_rng(8).choice([0, 1, 5], size=(2, 15, 12, 18), p=[0.3, 0.6, 0.1])
+    cls, ocls = ((tau.PeriodicElectrodeSolver, OraclePeriodicElectrodeSolver) if periodic else
+                 (tau.ElectrodeSolver, OracleElectrodeSolver))
+    _same(cls(img, spacing=0.5), ocls(img, spacing=0.5), 109)
+
+
+@pytest.mark.parametrize("cls,ocls", [(tau.Solver, OracleSolver), (tau.PeriodicSolver, OraclePeriodicSolver)])
+def test_a_wait_that_runs_out(cls, ocls):
+    """With a single poll per wait the exchange is lost; the iterations are
+    repeated by the streaming sweep and end on the same field."""
+    img = _binary((40, 44, 46), 6)
+    s = cls(img)
+    assert s._resident_sweep()
+    s._resident.spin = 1
+    s.solve(iter_limit=330, verbose=False, conv_crit=0.0)
+    assert np.array_equal(s.field.cpu().numpy(), ocls(img).run(330).field.numpy())
+    s.reset()
+    s.solve(iter_limit=230, verbose=False, conv_crit=0.0)
+    assert np.array_equal(s.field.cpu().numpy(), ocls(img).run(230).field.numpy())
+
+
+def test_tiny_values_take_the_division():
+    """Subnormal and tiny fields: the quotients the reciprocal does not give."""
+    img = _binary((12, 10, 70), 9, p=0.8)
+    for cls, ocls, extra in ((tau.Solver, OracleSolver, ()), (tau.AnisotropicSolver, OracleAnisotropicSolver,
+                                                             ((1.0, 1.2, 0.7),)),
+                             (tau.ElectrodeSolver, OracleElectrodeSolver, ())):
+        s, o = cls(img, *extra), ocls(img, *extra)
+        rng = np.random.default_rng(2)
+        f = o.field.numpy().copy()
+        tiny = np.ldexp(rng.standard_normal(f.shape), rng.integers(-149, -95, f.shape)).astype(np.float32)
+        f[:, 1:-1, 1:-1, 1:-1] = tiny[:, 1:-1, 1:-1, 1:-1] * (f[:, 1:-1, 1:-1, 1:-1] != 0)
+        f[:, [0, -1]] = 0.0  # nothing large flows in
+        o.field = torch.from_numpy(f.copy())
+        s.field = torch.from_numpy(f)
+        _same(s, o, 11)
