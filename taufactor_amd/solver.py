@@ -24,6 +24,7 @@ from __future__ import annotations
 import ctypes
 
 import math
+import threading
 import warnings
 from abc import ABC, abstractmethod
 from timeit import default_timer as timer
@@ -589,6 +590,13 @@ class SORSolver(ABC):
                   f"{torch.cuda.max_memory_reserved(device=self.device) / 1e6:.2f} MB reserved)")
 
 
+# the stream of the latest resident launch of each device: two of them at once
+# would wait for each other's compute units until their waits run out, so one
+# on another stream is ordered after it
+_resident_turn: dict = {}
+_resident_lock = threading.Lock()
+
+
 class _ResidentSweep:
     """The resident sweep of one solver (tf_sweep_resident): its layout,
     mailbox and the launches not yet known to have run to their end."""
@@ -627,10 +635,16 @@ class _ResidentSweep:
         if ev is not None:
             t0, t1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
             t0.record()
-        st = s._lib.tf_sweep_resident(_lib.ptr(src), _lib.ptr(dst), codes, table, self.kind, s.batch_size, s.Nx,
-                                      s.Ny, s.Nz, s._w32, it & 1, n, self.plan, _lib.ptr(self.mail),
-                                      self.plan.mail_bytes, self.tag, _lib.ptr(self.status), self.count, self.spin,
-                                      s._stream())
+        stream = torch.cuda.current_stream(s.device)
+        with _resident_lock:
+            last = _resident_turn.get(s.device.index)
+            if last is not None and last != stream:
+                stream.wait_event(last.record_event())
+            st = s._lib.tf_sweep_resident(_lib.ptr(src), _lib.ptr(dst), codes, table, self.kind, s.batch_size, s.Nx,
+                                          s.Ny, s.Nz, s._w32, it & 1, n, self.plan, _lib.ptr(self.mail),
+                                          self.plan.mail_bytes, self.tag, _lib.ptr(self.status), self.count,
+                                          self.spin, stream.cuda_stream)
+            _resident_turn[s.device.index] = stream
         if st == _lib.NOT_RESIDENT and not self.log:
             s._resident = False
             return False

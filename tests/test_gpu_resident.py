@@ -118,3 +118,27 @@ def test_tiny_values_take_the_division():
         o.field = torch.from_numpy(f.copy())
         s.field = torch.from_numpy(f)
         _same(s, o, 11)
+
+
+def test_streams_take_turns():
+    """Solvers on streams of their own, in threads: their resident launches
+    wait for each other's end on the device, none runs out of its waits."""
+    import threading
+
+    imgs = [_binary((120, 110, 100), i) for i in range(3)]
+    solvers = [None] * len(imgs)
+
+    def work(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            s = solvers[i] = tau.Solver(imgs[i])
+            s.solve(iter_limit=310, verbose=False, conv_crit=0.0)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(imgs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for s, img in zip(solvers, imgs):
+        assert s._resident
+        assert np.array_equal(s.field.cpu().numpy(), OracleSolver(img).run(310).field.numpy())
