@@ -37,7 +37,7 @@
 extern "C" {
 #endif
 
-#define TF_ABI_VERSION 13
+#define TF_ABI_VERSION 14
 
 #define TF_KIND_SOLVER 0
 #define TF_KIND_MULTIPHASE 1
@@ -473,6 +473,14 @@ int tf_spans_x(const uint8_t* mask, int X, int Y, int Z);
  * calibrates the HBM traffic counters and gives the device's copy rate
  * against which the sweep's measured traffic is read.                    */
 int tf_hbm_copy(const void* src, void* dst, long long bytes, void* stream);
+
+/* Host: input impedance of bs transmission lines of nx resistors R and
+ * capacitors C (both [bs][nx]) at nf frequencies each ([bs][nf]), from the
+ * closed right end: Z <- R_i + 1/(j w C_i + 1/Z), Z = 1e50 at first.  Replaces
+ * compute_impedance_batched (taufactor/utils.py:87-98).
+ *   out   complex [bs][nf] as (re, im) pairs */
+int tf_impedance(const double* R, const double* C, const double* freq, int bs, int nx, int nf,
+                 double* out);
 
 /* Resident sweep: a volume that fits into the registers of the device at
  * once, any number of half-sweeps in one launch (same iterates as tf_sweep).

@@ -17,7 +17,6 @@ import torch
 
 from . import _lib
 from .solver import SORSolver, _PeriodicYZ
-from .utils import compute_impedance_batched
 
 __all__ = ["ElectrodeSolver", "PeriodicElectrodeSolver"]
 
@@ -106,6 +105,16 @@ class ElectrodeSolver(SORSolver):
         return torch.gather(self._hm_lut, 1, c.reshape(self.batch_size, -1)).reshape(c.shape)
 
     # ---------------- metrics ----------------
+    def _impedance(self, R, C, freq):
+        """compute_impedance_batched (taufactor/utils.py:87-98) of float64
+        [B, X] resistors and capacitors at [B, F] frequencies, natively."""
+        R, C, freq = (np.ascontiguousarray(a, dtype=np.float64) for a in (R, C, freq))
+        out = np.empty(freq.shape, dtype=complex)
+        st = self._lib.tf_impedance(R.ctypes.data, C.ctypes.data, freq.ctypes.data, R.shape[0], R.shape[1],
+                                    freq.shape[1], out.ctypes.data)
+        _lib.check(st, "tf_impedance")
+        return out
+
     def compute_metrics(self):
         """taufactor/electrode.py:72-104, from float64 per-layer sums."""
         flux_sum, conc_sum = self._layer_sums()
@@ -131,10 +140,10 @@ class ElectrodeSolver(SORSolver):
         R = self.tau_x / eps
         R[eps == 0] = 1e30
         R[np.isnan(self.tau_x)] = 1e30
-        self.Z_sim = compute_impedance_batched(R, a_dx, freq)
+        self.Z_sim = self._impedance(R, a_dx, freq)
         R_ideal = 1 / np.mean(eps, axis=1)[:, None].repeat(self.Nx, axis=1)
         C_ideal = np.mean(a_dx, axis=1)[:, None].repeat(self.Nx, axis=1)
-        self.Z_ideal = compute_impedance_batched(R_ideal, C_ideal, freq)
+        self.Z_ideal = self._impedance(R_ideal, C_ideal, freq)
         tau = self.Z_sim[:, 0].real / self.Z_ideal[:, 0].real
         return tau, relative_error
 

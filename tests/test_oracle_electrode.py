@@ -74,3 +74,27 @@ def test_impedance_recurrence_matches_nodal_analysis(n):
     np.testing.assert_allclose(compute_impedance(R[0], C[0], freq), want[0], rtol=1e-9)
     # at high frequency the first capacitor shorts the rest of the line: Z -> R_0
     assert abs(compute_impedance(R[0], C[0], np.array([1e9]))[0] - R[0, 0]) < 1e-6
+
+
+@pytest.mark.parametrize("n", [1, 2, 57])
+def test_native_impedance_matches_numpy(n):
+    """tf_impedance against the numpy recurrence: ordinary lines, lines with
+    broken layers (R = 1e30) and no capacitors, an infinite frequency."""
+    from taufactor_amd import _lib
+    from taufactor_amd.utils import compute_impedance_batched
+
+    rng = np.random.default_rng(n)
+    R = rng.uniform(0.5, 3.0, size=(4, n))
+    C = rng.uniform(0.1, 2.0, size=(4, n))
+    R[1, n // 2] = 1e30
+    C[2, :] = 0.0
+    w = np.array([[1e-4, 3.0], [0.2, 1e6], [0.5, 1.0], [np.inf, 1e-9]])
+    out = np.empty((4, 2), dtype=complex)
+    st = _lib.load().tf_impedance(R.ctypes.data, C.ctypes.data, w.ctypes.data, 4, n, 2, out.ctypes.data)
+    assert st == 0
+    with np.errstate(all="ignore"):
+        want = compute_impedance_batched(R, C, w)
+    fin = np.isfinite(w)
+    # a chain of n correctly scaled divisions: a few ulp per layer
+    np.testing.assert_allclose(out[fin], want[fin], rtol=1e-15 * 8 * (n + 1))
+    assert _lib.load().tf_impedance(None, C.ctypes.data, w.ctypes.data, 4, n, 2, out.ctypes.data) < 0
