@@ -37,7 +37,7 @@
 extern "C" {
 #endif
 
-#define TF_ABI_VERSION 14
+#define TF_ABI_VERSION 15
 
 #define TF_KIND_SOLVER 0
 #define TF_KIND_MULTIPHASE 1
@@ -473,6 +473,15 @@ int tf_spans_x(const uint8_t* mask, int X, int Y, int Z);
  * calibrates the HBM traffic counters and gives the device's copy rate
  * against which the sweep's measured traffic is read.                    */
 int tf_hbm_copy(const void* src, void* dst, long long bytes, void* stream);
+
+/* Checks B maps of n voxel diffusivities (float32, device) and sums them:
+ * *bad (device int, set by the call) is 1 if any value is negative or not
+ * finite, part[b][i], i < TF_FIELD_PARTS, the float64 partial sums of map b
+ * (their sum in this order does not depend on scheduling).  No reference
+ * counterpart: the host checks of FieldSolver on a map that lives on the
+ * device. */
+#define TF_FIELD_PARTS 256
+int tf_field_stats(const float* k, int B, long long n, double* part, int* bad, void* stream);
 
 /* Host: input impedance of bs transmission lines of nx resistors R and
  * capacitors C (both [bs][nx]) at nf frequencies each ([bs][nf]), from the

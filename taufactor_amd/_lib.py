@@ -11,7 +11,7 @@ import threading
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libtauhip.so")
-ABI_VERSION = 14
+ABI_VERSION = 15
 
 KIND_SOLVER = 0
 KIND_MULTIPHASE = 1
@@ -23,6 +23,7 @@ KIND_MULTIPHASE_FACES = 5
 MPF_MAX_CLASSES = 4
 MPF_FACE_SLOTS = 16
 MPF_MAX_FACTORS = 2047
+FIELD_PARTS = 256  # partial sums per map of tf_field_stats
 SWEEP_PERIODIC_YZ = 0x100  # flag OR-ed into the kind of tf_sweep
 ELECTRODE_TABLE = 64
 SETUP_PERIODIC_YZ = 1
@@ -82,6 +83,7 @@ SIGNATURES = {
     "tf_layer_sums_noalloc": (_c_int, [_vp, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                                        _vp, _vp, _vp]),
     "tf_spans_x": (_c_int, [_vp, _c_int, _c_int, _c_int]),
+    "tf_field_stats": (_c_int, [_vp, _c_int, ctypes.c_longlong, _vp, _vp, _vp]),
     "tf_impedance": (_c_int, [_vp, _vp, _vp, _c_int, _c_int, _c_int, _vp]),
     "tf_setup_field": (_c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _vp]),
     "tf_field_faces": (_c_int, [_vp, _vp, _c_int, _c_int, _c_int, _c_int, _vp]),

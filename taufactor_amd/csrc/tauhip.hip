@@ -1259,6 +1259,51 @@ extern "C" int tf_setup_field(const float* k, const float* xinit, float* kpad, f
     return 0;
 }
 
+// Validity and float64 sum of the voxel diffusivities: block i of a volume
+// takes every TF_FIELD_PARTS-th chunk of 1024 voxels.  Bound: HBM (4 B per
+// voxel, read once); 4 x 128^3 take 13 us, where copying the map to the host
+// and looking through it there took 19 ms.
+constexpr int kStatThreads = 256, kStatPer = 4;
+__global__ __launch_bounds__(kStatThreads) void k_field_stats(const float* __restrict__ k, long long n,
+                                                              double* __restrict__ part, int* __restrict__ bad) {
+    const float* K = k + (size_t)blockIdx.y * n;
+    const long long step = (long long)gridDim.x * kStatThreads * kStatPer;
+    double acc = 0.0;
+    bool ok = true;
+    for (long long i0 = (long long)blockIdx.x * kStatThreads * kStatPer + threadIdx.x; i0 < n; i0 += step) {
+        float f[kStatPer];
+#pragma unroll
+        for (int j = 0; j < kStatPer; ++j) f[j] = i0 + j * kStatThreads < n ? K[i0 + j * kStatThreads] : 0.0f;
+#pragma unroll
+        for (int j = 0; j < kStatPer; ++j) {
+            ok = ok && f[j] >= 0.0f && f[j] < __builtin_inff();
+            acc += (double)f[j];
+        }
+    }
+    __shared__ double red[kStatThreads / 64];
+    for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+    if (!ok) *bad = 1;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double s = red[0];
+        for (int i = 1; i < kStatThreads / 64; ++i) s += red[i];
+        part[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = s;
+    }
+}
+
+__global__ void k_clear_flag(int* flag) { *flag = 0; }
+
+extern "C" int tf_field_stats(const float* k, int B, long long n, double* part, int* bad, void* stream) {
+    if (!k || !part || !bad) return fail(-1, "null pointer argument");
+    if (B < 1 || B > kMaxGridY || n < 1) return fail(-1, "invalid shape B=%d n=%lld", B, n);
+    hipStream_t st = (hipStream_t)stream;
+    hipLaunchKernelGGL(k_clear_flag, dim3(1), dim3(1), 0, st, bad);
+    hipLaunchKernelGGL(k_field_stats, dim3(TF_FIELD_PARTS, B), dim3(kStatThreads), 0, st, k, n, part, bad);
+    TF_LAUNCH_CHECK("k_field_stats");
+    return 0;
+}
+
 // Face conductances of the per-voxel field for the sweep: for every padded
 // voxel o, gx[o] = hm(k[o], k[o + x]), gy[o] = hm(k[o], k[o + y]),
 // gz[o] = hm(k[o], k[o + z]) (0 where the neighbour is outside the padded

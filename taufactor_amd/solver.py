@@ -60,8 +60,7 @@ class SORSolver(ABC):
     _zero_yz_ghosts: bool = True  # closed y/z boundaries: the ghosts stay 0
 
     def __init__(self, img: np.ndarray, omega: float | None = None, precision=None, device="cuda"):
-        self.cpu_img = self._expand_to_4d(img)
-        self.batch_size, self.Nx, self.Ny, self.Nz = self.cpu_img.shape
+        self.batch_size, self.Nx, self.Ny, self.Nz = self._take_image(img)
         self.device = self._init_device(device)
         self.precision = precision or torch.float
         if self.precision != torch.float32:
@@ -549,6 +548,11 @@ class SORSolver(ABC):
             return self.tau_x
 
     # ---------------- helpers ----------------
+    def _take_image(self, img):
+        """Keep the input image; returns its four extents."""
+        self.cpu_img = self._expand_to_4d(img)
+        return self.cpu_img.shape
+
     @staticmethod
     def _expand_to_4d(img: np.ndarray) -> np.ndarray:
         if not isinstance(img, np.ndarray):
@@ -1243,15 +1247,59 @@ class FieldSolver(ThroughTransportSolver):
 
     def __init__(self, k, D_scaling=1, omega=None, device="cuda"):
         self._k_tensor = k if isinstance(k, torch.Tensor) else None
-        k_np = k.detach().cpu().numpy() if isinstance(k, torch.Tensor) else k
-        if not isinstance(k_np, np.ndarray):
-            raise TypeError("Error: input image must be a NumPy array!")
-        if k_np.size and (not np.all(np.isfinite(k_np)) or k_np.min() < 0):
-            raise ValueError("voxel diffusivities must be finite and >= 0")
+        self._cpu_img = None
+        self._k_mean = None
+        if self._k_tensor is not None and self._on_device(k, device):
+            img = k.detach()  # checked and summed where it is
+        else:
+            img = k.detach().cpu().numpy() if isinstance(k, torch.Tensor) else k
+            if not isinstance(img, np.ndarray):
+                raise TypeError("Error: input image must be a NumPy array!")
+            if img.size and (not np.all(np.isfinite(img)) or img.min() < 0):
+                raise ValueError("voxel diffusivities must be finite and >= 0")
         self.conductive_labels = None
-        super().__init__(k_np, omega=omega, device=device)
+        super().__init__(img, omega=omega, device=device)
         self.D_0 = D_scaling
-        self.D_mean = self.cpu_img.reshape(self.batch_size, -1).astype(np.float32).astype(np.float64).mean(axis=1)
+        self.D_mean = self._k_mean if self._k_mean is not None else \
+            self.cpu_img.reshape(self.batch_size, -1).astype(np.float32).astype(np.float64).mean(axis=1)
+
+    @classmethod
+    def _on_device(cls, k, device) -> bool:
+        """A float32 map already on the solver's device (and not empty)."""
+        return k.is_cuda and k.dtype == torch.float32 and k.numel() > 0 and 2 <= k.dim() <= 4 \
+            and k.shape[0] <= 65535 and k.device == cls._init_device(device)
+
+    def _take_image(self, img):
+        if isinstance(img, np.ndarray):
+            return super()._take_image(img)
+        t = img[..., None] if img.dim() == 2 else img
+        t = t[None, ...] if t.dim() == 3 else t
+        B, n = t.shape[0], t[0].numel()
+        with torch.cuda.device(t.device):
+            t = t.contiguous()
+            buf = torch.empty(B * _lib.FIELD_PARTS + 1, dtype=torch.float64, device=t.device)
+            lib = _lib.load()
+            st = lib.tf_field_stats(_lib.ptr(t), B, n, _lib.ptr(buf), _lib.ptr(buf) + 8 * B * _lib.FIELD_PARTS,
+                                    _lib.stream_handle(t.device))
+            _lib.check(st, "tf_field_stats")
+            h = buf.cpu().numpy()
+        if h[-1:].view(np.int32)[0]:
+            raise ValueError("voxel diffusivities must be finite and >= 0")
+        self._k_mean = h[:-1].reshape(B, -1).sum(axis=1) / n
+        self._k_tensor = t
+        return tuple(t.shape)
+
+    @property
+    def cpu_img(self):
+        """The voxel diffusivities on the host, [B, X, Y, Z] (of a map that
+        was given on the device: copied back when first asked for)."""
+        if self._cpu_img is None:
+            self._cpu_img = self._codes[:, 1:-1, 1:-1, 1:-1].cpu().numpy()
+        return self._cpu_img
+
+    @cpu_img.setter
+    def cpu_img(self, value):
+        self._cpu_img = value
 
     def _spans(self, b):
         if b not in self._spans_cache:
