@@ -37,7 +37,7 @@
 extern "C" {
 #endif
 
-#define TF_ABI_VERSION 15
+#define TF_ABI_VERSION 16
 
 #define TF_KIND_SOLVER 0
 #define TF_KIND_MULTIPHASE 1
@@ -106,6 +106,9 @@ typedef struct tf_resident {
     long long mail_bytes;
 } tf_resident;
 
+/* the longest face-code table (n_classes of TF_KIND_MULTIPHASE_FACES) of the
+ * resident sweep */
+#define TF_RESIDENT_TABLE 508
 /* status of tf_sweep_resident: the device cannot hold the workgroups at once */
 #define TF_NOT_RESIDENT (-2)
 
@@ -483,6 +486,13 @@ int tf_hbm_copy(const void* src, void* dst, long long bytes, void* stream);
 #define TF_FIELD_PARTS 256
 int tf_field_stats(const float* k, int B, long long n, double* part, int* bad, void* stream);
 
+/* Face conductances of class codes (TF_KIND_MULTIPHASE's padded codes and
+ * n_classes x n_classes table) in the sections of tf_field_faces, as
+ * TF_KIND_FIELD reads them: gx, gy, gz of every padded voxel, zero past the
+ * padded volume. */
+int tf_class_faces(const uint8_t* codes, const float* hm_lut, int n_classes, float* faces, int B,
+                   int X, int Y, int Z, void* stream);
+
 /* Host: input impedance of bs transmission lines of nx resistors R and
  * capacitors C (both [bs][nx]) at nf frequencies each ([bs][nf]), from the
  * closed right end: Z <- R_i + 1/(j w C_i + 1/Z), Z = 1e50 at first.  Replaces
@@ -494,15 +504,17 @@ int tf_impedance(const double* R, const double* C, const double* freq, int bs, i
 /* Resident sweep: a volume that fits into the registers of the device at
  * once, any number of half-sweeps in one launch (same iterates as tf_sweep).
  *
- * tf_resident_plan chooses the layout for `kind` (TF_KIND_SOLVER,
- * TF_KIND_ANISOTROPIC or TF_KIND_ELECTRODE, optionally with
- * TF_SWEEP_PERIODIC_YZ) on a device of compute_units CUs: 1 and *plan if the
+ * tf_resident_plan chooses the layout for `kind` (TF_KIND_SOLVER or
+ * TF_KIND_ELECTRODE, optionally with TF_SWEEP_PERIODIC_YZ,
+ * TF_KIND_ANISOTROPIC, TF_KIND_FIELD or TF_KIND_MULTIPHASE_FACES) on a device of compute_units CUs: 1 and *plan if the
  * volume fits, 0 if it does not.  Host only.
  *
  * tf_sweep_resident runs n_half half-sweeps from src into dst (distinct, both
  * with their ghosts set; only the interior of dst is written).
- *   codes     the sweep codes, as tf_sweep
- *   table     as hm_lut of tf_sweep (null for TF_KIND_SOLVER)
+ *   codes     as tf_sweep: the sweep codes, the face sections (`section`
+ *             floats apart, at least B volumes) or the face codes
+ *   table     as hm_lut of tf_sweep (null for TF_KIND_SOLVER, TF_KIND_FIELD),
+ *             n_table floats (face codes: at most TF_RESIDENT_TABLE)
  *   mail      plan->mail_bytes of 8-byte aligned device memory, zero before
  *             the first launch, used by one launch at a time
  *   tag       counts the half-sweeps of all launches on this mailbox: at
@@ -514,10 +526,11 @@ int tf_impedance(const double* R, const double* C, const double* freq, int bs, i
  * TF_NOT_RESIDENT if the device cannot hold the workgroups at once (nothing
  * is launched). */
 int tf_resident_plan(int kind, int B, int X, int Y, int Z, int compute_units, tf_resident* plan);
-int tf_sweep_resident(const float* src, float* dst, const uint8_t* codes, const float* table,
-                      int kind, int B, int X, int Y, int Z, float omega, int first_colour,
-                      int n_half, const tf_resident* plan, void* mail, long long mail_bytes,
-                      uint32_t tag, int* status, int launch_id, int spin, void* stream);
+int tf_sweep_resident(const float* src, float* dst, const void* codes, const float* table,
+                      int n_table, int kind, int B, int X, int Y, int Z, float omega,
+                      int first_colour, int n_half, const tf_resident* plan, long long section,
+                      void* mail, long long mail_bytes, uint32_t tag, int* status, int launch_id,
+                      int spin, void* stream);
 
 #ifdef __cplusplus
 }

@@ -11,7 +11,7 @@ import threading
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libtauhip.so")
-ABI_VERSION = 15
+ABI_VERSION = 16
 
 KIND_SOLVER = 0
 KIND_MULTIPHASE = 1
@@ -48,6 +48,8 @@ class Resident(ctypes.Structure):
         [("mail_bytes", ctypes.c_longlong)]
 
 
+# longest face-code table of the resident sweep (TF_RESIDENT_TABLE)
+RESIDENT_TABLE = 508
 # status of tf_sweep_resident: the device cannot hold the workgroups at once
 NOT_RESIDENT = -2
 
@@ -70,9 +72,10 @@ SIGNATURES = {
     "tf_sweep": (_c_int, [_vp, _vp, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                           _c_float, _c_int, _c_int, ctypes.POINTER(Tile), _vp]),
     "tf_resident_plan": (_c_int, [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, ctypes.POINTER(Resident)]),
-    "tf_sweep_resident": (_c_int, [_vp, _vp, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int,
-                                   _c_int, ctypes.POINTER(Resident), _vp, ctypes.c_longlong, ctypes.c_uint32, _vp,
-                                   _c_int, _c_int, _vp]),
+    "tf_sweep_resident": (_c_int, [_vp, _vp, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float,
+                                   _c_int, _c_int, ctypes.POINTER(Resident), ctypes.c_longlong, _vp,
+                                   ctypes.c_longlong, ctypes.c_uint32, _vp, _c_int, _c_int, _vp]),
+    "tf_class_faces": (_c_int, [_vp, _vp, _c_int, _vp, _c_int, _c_int, _c_int, _c_int, _vp]),
     "tf_sweep_half_inplace": (_c_int, [_vp, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_int,
                                        _c_int, _c_float, _c_int, _vp]),
     "tf_layer_sums": (_c_int, [_vp, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,

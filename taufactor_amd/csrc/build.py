@@ -18,7 +18,8 @@ ROOT = os.path.dirname(PKG)
 # parallel: the sweep templates dominate the build)
 SOURCES = ["tauhip.hip", "sweep_solver.hip", "sweep_multiphase.hip", "sweep_mpfaces.hip", "sweep_field.hip",
            "sweep_anisotropic.hip", "sweep_electrode.hip", "sweep_batch.hip",
-           "resident_solver.hip", "resident_periodic.hip", "resident_anisotropic.hip", "resident_electrode.hip"]
+           "resident_solver.hip", "resident_periodic.hip", "resident_anisotropic.hip", "resident_electrode.hip",
+           "resident_field.hip", "resident_mpfaces.hip"]
 INCLUDE = os.path.join(ROOT, "include")
 OUT = os.path.join(PKG, "libtauhip.so")
 OBJ_DIR = os.path.join(HERE, "_build")

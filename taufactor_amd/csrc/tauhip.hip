@@ -597,13 +597,33 @@ extern "C" int tf_sweep_launch_config(int kind, int n_classes, int B, int X, int
 // ---------------------------------------------------------------------------
 struct ResidentShapeDesc {
     int elems, px, py, waves;
-    size_t (*lds_floats)(int wy);  // of the kind with the largest table
+    size_t (*lds_floats)(int wy);  // (code kinds: with the largest table)
 };
-static const ResidentShapeDesc kResidentShapes[] = {
-#define F(P, PX, PY, NW) {P, PX, PY, NW, ResidentShape<TF_KIND_ANISOTROPIC, P, PX, PY, NW>::lds_floats},
-    TF_RESIDENT_SHAPES(F)
+template <int KIND>
+static const std::vector<ResidentShapeDesc>& resident_shapes_of() {
+#define F(P, PX, PY, NW) {P, PX, PY, NW, ResidentShape<KIND, P, PX, PY, NW>::lds_floats},
+    if constexpr (KIND == TF_KIND_FIELD) {
+        static const std::vector<ResidentShapeDesc> v = {TF_RESIDENT_SHAPES_FIELD(F)};
+        return v;
+    } else if constexpr (KIND == TF_KIND_MULTIPHASE_FACES) {
+        static const std::vector<ResidentShapeDesc> v = {TF_RESIDENT_SHAPES_FACES(F)};
+        return v;
+    } else {
+        static const std::vector<ResidentShapeDesc> v = {TF_RESIDENT_SHAPES(F)};
+        return v;
+    }
 #undef F
-};
+}
+static const std::vector<ResidentShapeDesc>& resident_shapes(int kind) {
+    return kind == TF_KIND_FIELD               ? resident_shapes_of<TF_KIND_FIELD>()
+           : kind == TF_KIND_MULTIPHASE_FACES ? resident_shapes_of<TF_KIND_MULTIPHASE_FACES>()
+                                              : resident_shapes_of<TF_KIND_ANISOTROPIC>();
+}
+
+static long long resident_mail_bytes(const ResidentShapeDesc& s, int wy, long long tiles) {
+    const long long rows = 2LL * (wy * s.py + s.waves / wy * s.px);
+    return tiles * 2 * rows * (s.elems / 2) * 64 * 8;
+}
 
 // Geometry of one shape with wx x wy waves; false if the volume does not fit
 // it.  A wave asks for at most one face per axis from another workgroup
@@ -621,17 +641,15 @@ static bool resident_geometry(const ResidentShapeDesc& s, int wy, int B, int X, 
     if (*ntx > 1 && wx < 2) return false;
     if (*nty > 1 && wy < 2) return false;
     if (periodic && *nty > 1 && ngy % wy == 1) return false;
-    return *ntx * *nty * B <= (1 << 20);
-}
-
-static long long resident_mail_bytes(const ResidentShapeDesc& s, int wy, long long tiles) {
-    const long long rows = 2LL * (wy * s.py + s.waves / wy * s.px);
-    return tiles * 2 * rows * (s.elems / 2) * 64 * 8;
+    const long long tiles = *ntx * *nty * B;
+    return tiles <= (1 << 20) && resident_mail_bytes(s, wy, tiles) < (1LL << 31);  // 32-bit offsets
 }
 
 static int resident_kind(int& kind, int& periodic, int Y, int Z) {
     if (int rc = split_sweep_kind(kind, periodic, Y, Z)) return rc;
-    if (!own_code_kind(kind)) return fail(-1, "no resident sweep of kind %d", kind);
+    if (kind == TF_KIND_FIELD || (kind == TF_KIND_MULTIPHASE_FACES && !periodic)) return 0;
+    if (!own_code_kind(kind))
+        return fail(-1, "no resident sweep of kind %d%s", kind, periodic ? " with periodic y/z" : "");
     return 0;
 }
 
@@ -644,7 +662,7 @@ extern "C" int tf_resident_plan(int kind, int B, int X, int Y, int Z, int comput
     const int lane_y = Z == 1 && Y > 1;
     const int lane_n = lane_y ? Y : Z, row_n = lane_y ? 1 : Y;
     long long best = -1, best_mail = 0;
-    for (const ResidentShapeDesc& s : kResidentShapes) {
+    for (const ResidentShapeDesc& s : resident_shapes(kind)) {
         // the fewest voxels per lane that cover a row
         if (lane_n > 64 * s.elems || (s.elems > 2 && lane_n <= 32 * s.elems)) continue;
         for (int wy = 1; wy <= s.waves; ++wy) {
@@ -665,14 +683,20 @@ extern "C" int tf_resident_plan(int kind, int B, int X, int Y, int Z, int comput
     return best >= 0 ? 1 : 0;
 }
 
-extern "C" int tf_sweep_resident(const float* src, float* dst, const uint8_t* codes, const float* table,
-                                 int kind, int B, int X, int Y, int Z, float omega, int first_colour,
-                                 int n_half, const tf_resident* plan, void* mail, long long mail_bytes,
-                                 uint32_t tag, int* status, int launch_id, int spin, void* stream) {
+extern "C" int tf_sweep_resident(const float* src, float* dst, const void* codes, const float* table,
+                                 int n_table, int kind, int B, int X, int Y, int Z, float omega,
+                                 int first_colour, int n_half, const tf_resident* plan, long long section,
+                                 void* mail, long long mail_bytes, uint32_t tag, int* status, int launch_id,
+                                 int spin, void* stream) {
     if (int rc = check_dims(B, X, Y, Z)) return rc;
     int periodic = 0;
     if (int rc = resident_kind(kind, periodic, Y, Z)) return rc;
-    if (!src || !dst || !codes || !plan || !mail || !status || (kind != TF_KIND_SOLVER && !table))
+    if (kind == TF_KIND_MULTIPHASE_FACES && (n_table < TF_MPF_FACE_SLOTS + 2 || n_table > TF_RESIDENT_TABLE))
+        return fail(-1, "face-code table of %d floats out of range", n_table);
+    if (kind == TF_KIND_FIELD && section < (long long)B * make_vol(X, Y, Z).sB)
+        return fail(-1, "face sections of %lld floats do not hold the volumes", section);
+    if (!src || !dst || !codes || !plan || !mail || !status ||
+        (kind != TF_KIND_SOLVER && kind != TF_KIND_FIELD && !table))
         return fail(-1, "null pointer argument");
     if (src == dst) return fail(-1, "tf_sweep_resident needs distinct src and dst buffers");
     if (first_colour != 0 && first_colour != 1) return fail(-1, "first_colour must be 0 or 1");
@@ -701,7 +725,8 @@ extern "C" int tf_sweep_resident(const float* src, float* dst, const uint8_t* co
     const long long need = resident_mail_bytes(s, plan->wy, a.total);
     if (mail_bytes < need || ((uintptr_t)mail & 7))
         return fail(-1, "a mailbox of %lld 8-byte aligned bytes is needed (got %lld)", need, mail_bytes);
-    a.src = src; a.dst = dst; a.codes = codes; a.table = table;
+    a.src = src; a.dst = dst; a.codes = codes; a.table = table; a.n_table = n_table;
+    a.fsec = section;
     a.w = omega;
     a.colour0 = first_colour;
     a.n_half = n_half;
@@ -712,6 +737,8 @@ extern "C" int tf_sweep_resident(const float* src, float* dst, const uint8_t* co
     a.launch_id = launch_id;
     a.spin = spin > 0 ? spin : kResidentSpin;
     const hipStream_t st = (hipStream_t)stream;
+    if (kind == TF_KIND_FIELD) return resident_dispatch_field(*plan, a, st);
+    if (kind == TF_KIND_MULTIPHASE_FACES) return resident_dispatch_mpfaces(*plan, a, st);
     if (kind == TF_KIND_ANISOTROPIC) return resident_dispatch_anisotropic(*plan, a, st);
     if (kind == TF_KIND_ELECTRODE) return resident_dispatch_electrode(*plan, a, periodic, st);
     return periodic ? resident_dispatch_periodic(*plan, a, st) : resident_dispatch_solver(*plan, a, st);
@@ -1341,6 +1368,42 @@ extern "C" int tf_field_faces(const float* kpad, float* faces, int B, int X, int
         hipLaunchKernelGGL(k_field_faces, dim3(gx, (unsigned)min(B - b0, kMaxGridY)), dim3(kSetupThreads), 0,
                            (hipStream_t)stream, kpad, faces, v, b0, nbx, total);
         TF_LAUNCH_CHECK("k_field_faces");
+    }
+    return 0;
+}
+
+// The same sections for class codes: gx[o] = hm[c[o]][c[o + x]] and so on from
+// the n_classes x n_classes face-conductance table, for the resident sweep
+// of class-coded volumes (the values that TF_KIND_MULTIPHASE looks up).
+__global__ void k_class_faces(const uint8_t* __restrict__ C, const float* __restrict__ hm, int ncls,
+                              float* __restrict__ faces, Vol v, int b0, int nbx, long long fsec) {
+    const int xp = (int)(blockIdx.x / (unsigned)nbx);
+    const int r2 = (int)(blockIdx.x - (unsigned)xp * (unsigned)nbx) * (int)blockDim.x + (int)threadIdx.x;
+    if (r2 >= v.sX) return;
+    const int yp = r2 / v.sY, zp = r2 - yp * v.sY;
+    const size_t o = (size_t)(b0 + (int)blockIdx.y) * v.sB + (size_t)xp * v.sX + r2;
+    const bool xq = xp <= v.X, yq = yp <= v.Y, zq = zp <= v.Z;
+    const uint8_t* P = C + o;
+    const int c = P[0] * ncls, cx = P[xq ? v.sX : 0], cy = P[yq ? v.sY : 0], cz = P[zq ? 1 : 0];
+    faces[o] = xq ? hm[c + cx] : 0.0f;
+    faces[fsec + o] = yq ? hm[c + cy] : 0.0f;
+    faces[2 * fsec + o] = zq ? hm[c + cz] : 0.0f;
+}
+
+extern "C" int tf_class_faces(const uint8_t* codes, const float* hm_lut, int n_classes, float* faces, int B,
+                              int X, int Y, int Z, void* stream) {
+    if (int rc = check_dims(B, X, Y, Z)) return rc;
+    if (!codes || !hm_lut || !faces) return fail(-1, "null pointer argument");
+    if (n_classes < 1 || n_classes > 256) return fail(-1, "n_classes=%d out of range", n_classes);
+    const Vol v = make_vol(X, Y, Z);
+    int nbx;
+    unsigned gx;
+    if (int rc = set_up_grid(v, &nbx, &gx)) return rc;
+    for (int b0 = 0; b0 < B; b0 += kMaxGridY) {
+        hipLaunchKernelGGL(k_class_faces, dim3(gx, (unsigned)min(B - b0, kMaxGridY)), dim3(kSetupThreads), 0,
+                           (hipStream_t)stream, codes, hm_lut, n_classes, faces, v, b0, nbx,
+                           (long long)B * v.sB);
+        TF_LAUNCH_CHECK("k_class_faces");
     }
     return 0;
 }

@@ -47,8 +47,10 @@
 struct ResidentArgs {
     const float* src;
     float* dst;
-    const uint8_t* codes;  // sweep codes
-    const float* table;    // anisotropic, electrode: as for tf_sweep
+    const void* codes;     // as tf_sweep: sweep codes, face sections or face codes
+    const float* table;    // as tf_sweep
+    int n_table;           // face codes: its length
+    long long fsec;        // field kind: floats between the face sections
     Vol v;
     int lane_n, row_n;  // extents of the lane axis and the row axis
     int sL, sR;         // their strides in the padded volume
@@ -67,7 +69,10 @@ constexpr int kResidentSpin = 1 << 16;  // polls of one wait, about 50 ms
 
 template <int KIND>
 constexpr int resident_table_floats() {
-    return KIND == TF_KIND_SOLVER ? 18 : 2 * (KIND == TF_KIND_ELECTRODE ? TF_ELECTRODE_TABLE : TF_ANISO_TABLE);
+    return KIND == TF_KIND_SOLVER ? 18
+           : KIND == TF_KIND_FIELD ? 0
+           : KIND == TF_KIND_MULTIPHASE_FACES ? TF_RESIDENT_TABLE
+           : 2 * (KIND == TF_KIND_ELECTRODE ? TF_ELECTRODE_TABLE : TF_ANISO_TABLE);
 }
 
 template <int KIND, int P, int PX, int PY, int NW>
@@ -120,7 +125,11 @@ __global__ __launch_bounds__(NW * 64) void k_resident(ResidentArgs a) {
     constexpr int R = Sh::R, RB = Sh::RB, HP = Sh::HP, E = Sh::E, ROW = Sh::ROW, NBUF = Sh::NBUF, PUB = Sh::PUB;
     constexpr int NK = (E + 3) / 4;
     constexpr int kTable = resident_table_floats<KIND>();
-    constexpr bool kPairs = KIND != TF_KIND_SOLVER;
+    // per-voxel field: every face conductance in a register; MultiPhase face
+    // codes: a code word per voxel; the others: a code byte per voxel
+    constexpr bool kField = KIND == TF_KIND_FIELD, kFaceCodes = KIND == TF_KIND_MULTIPHASE_FACES;
+    constexpr bool kBytes = !kField && !kFaceCodes;
+    constexpr bool kPairs = KIND == TF_KIND_ANISOTROPIC || KIND == TF_KIND_ELECTRODE;
     static_assert(P % 2 == 0 && P >= 2, "a lane holds whole red/black pairs");
 
     // consecutive tiles on one XCD, as k_sweep
@@ -155,7 +164,9 @@ __global__ __launch_bounds__(NW * 64) void k_resident(ResidentArgs a) {
     for (int i = threadIdx.x; i < Sh::ZERO + Sh::face(a.WY); i += NW * 64) zero[i] = 0.0f;
     if constexpr (KIND == TF_KIND_SOLVER) {
         if (threadIdx.x < kTable) rs_smem[threadIdx.x] = c_rd[threadIdx.x];
-    } else {
+    } else if constexpr (kFaceCodes) {
+        for (int i = threadIdx.x; i < a.n_table; i += NW * 64) rs_smem[i] = a.table[i];
+    } else if constexpr (kPairs) {
         const float* tab = KIND == TF_KIND_ELECTRODE ? a.table + (size_t)b * TF_ELECTRODE_TABLE : a.table;
         for (int i = threadIdx.x; i < kTable / 2; i += NW * 64) {
             float r, f;
@@ -173,59 +184,91 @@ __global__ __launch_bounds__(NW * 64) void k_resident(ResidentArgs a) {
     // between the row's last voxel and the end of its last lane's elements
     // has code 0, so its value stays 0 whatever its neighbours hold.
     const float* const S = a.src + (size_t)b * a.v.sB;
-    const uint8_t* const C = a.codes + (size_t)b * sweep_code_volume(a.v.X, a.v.Y, a.v.Z);
     const int l0 = lane * P;
-    float F[R][P];
-    uint32_t K[NK];
+    // the lane's P words of the row whose first voxel is word o of `base`
+    auto load_row = [&](const float* base, size_t o, bool ok, float (&d)[P]) {
+        const rsrc_t r = make_rsrc(base + (ok ? o : 0), ok ? (uint32_t)((a.lane_n - 1) * a.sL + 1) * 4u : 0u);
+        const int vo = l0 * a.sL * 4;
+        if (a.sL == 1 && P == 2) {
+            const u32x2_t q = __builtin_amdgcn_raw_buffer_load_b64(r, vo, 0, 0);
+            d[0] = lo_f(q);
+            d[1] = hi_f(q);
+        } else if (a.sL == 1) {
+            typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 #pragma unroll
-    for (int i = 0; i < NK; ++i) K[i] = 0;
-    float wrow[PX];  // 0 in rows past the volume: a ghost row keeps its value
+            for (int e = 0; e + 3 < P; e += 4) {
+                const u32x4_t q = __builtin_amdgcn_raw_buffer_load_b128(r, vo + 4 * e, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const uint32_t u = q[i];
+                    d[e + i] = __builtin_bit_cast(float, u);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < P; ++e) d[e] = ld_f32(r, vo, e * a.sL * 4);
+        }
+    };
+    // word of voxel (x, r) of the patch's plane and row, the lane axis's first
+    auto word_at = [&](int x, int r) {
+        return (size_t)(x + 1) * a.v.sX + (size_t)(r + 1) * a.sR + a.sL;
+    };
+    float F[R][P];
+    uint32_t K[kBytes ? NK : 1];
+#pragma unroll
+    for (int i = 0; i < (kBytes ? NK : 1); ++i) K[i] = 0;
+    // the words of the voxels and of their neighbours on the minus sides,
+    // which hold those faces (lane axis: of the row's element before the
+    // lane's first)
+    constexpr int NS = kField ? 3 : kFaceCodes ? 1 : 0;  // words per voxel: x, row, lane faces
+    float G[NS > 0 ? NS : 1][R][P], Gx[PY][P], Gr[PX][P], Gl[R];
+    float wrow[PX];           // 0 in rows past the volume: a ghost row keeps its value
+    float first, last[PX];    // 1 in the first and the last layer (their x faces count twice)
+    const float* const W = kBytes ? S : reinterpret_cast<const float*>(a.codes) + (size_t)b * a.v.sB;
+    const float* const Wr = W + (kField ? (a.sL == 1 ? 1 : 2) * a.fsec : 0);  // row-axis faces
+    const float* const Wl = W + (kField ? (a.sL == 1 ? 2 : 1) * a.fsec : 0);  // lane-axis faces
+    first = gx == 0 ? 1.0f : 0.0f;
 #pragma unroll
     for (int ix = 0; ix < PX; ++ix) {
         const int x = gx * PX + ix;
         wrow[ix] = x < a.v.X ? a.w : 0.0f;
+        last[ix] = x == a.v.X - 1 ? 1.0f : 0.0f;
 #pragma unroll
         for (int iy = 0; iy < PY; ++iy) {
             const int r = gy * PY + iy, row = ix * PY + iy;
-            const bool ok = live && x <= a.v.X && r < a.row_n;
-            const size_t o = ok ? (size_t)(x + 1) * a.v.sX + (size_t)(r + 1) * a.sR + a.sL : 0;
-            const rsrc_t rF = make_rsrc(S + o, ok ? (uint32_t)((a.lane_n - 1) * a.sL + 1) * 4u : 0u);
-            const bool cok = ok && x < a.v.X;
-            // byte z + 3 of a code row is voxel z, the lane axis's first voxel z = 1
-            const size_t oc = cok ? (size_t)(x + 1) * a.cX + (size_t)(r + 1) * a.cR + (a.cL == 1 ? 4 : a.cL + 3) : 0;
-            // (codes along z: up to the end of the row's last word, zeros past Z)
-            const uint32_t nc = a.cL == 1 ? (uint32_t)a.cR - 4u : (uint32_t)((a.lane_n - 1) * a.cL + 1);
-            const rsrc_t rC = make_rsrc(C + oc, cok ? nc : 0u);
-            const int vo = l0 * a.sL * 4, vc = l0 * a.cL;
-            if (a.sL == 1 && P == 2) {
-                const u32x2_t q = __builtin_amdgcn_raw_buffer_load_b64(rF, vo, 0, 0);
-                F[row][0] = lo_f(q);
-                F[row][1] = hi_f(q);
-            } else if (a.sL == 1) {
-                typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-#pragma unroll
-                for (int e = 0; e + 3 < P; e += 4) {
-                    const u32x4_t q = __builtin_amdgcn_raw_buffer_load_b128(rF, vo + 4 * e, 0, 0);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const uint32_t u = q[i];
-                        F[row][e + i] = __builtin_bit_cast(float, u);
-                    }
+            const bool ok = live && x <= a.v.X && r < a.row_n, in = ok && x < a.v.X;
+            load_row(S, word_at(x, r), ok, F[row]);
+            if constexpr (NS > 0) {
+                load_row(W, word_at(x, r), in, G[0][row]);
+                if constexpr (kField) {
+                    load_row(Wr, word_at(x, r), in, G[1][row]);
+                    load_row(Wl, word_at(x, r), in, G[2][row]);
                 }
+                const size_t o = in ? word_at(x, r) - a.sL : 0;
+                Gl[row] = ld_f32(make_rsrc(Wl + o, in ? (uint32_t)((a.lane_n - 1) * a.sL + 1) * 4u : 0u), l0 * a.sL * 4);
+                if (ix == 0) load_row(W, word_at(x - 1, r), in, Gx[iy]);
+                if (iy == 0) load_row(Wr, word_at(x, r - 1), in, Gr[ix]);
             } else {
+                const uint8_t* const C =
+                    reinterpret_cast<const uint8_t*>(a.codes) + (size_t)b * sweep_code_volume(a.v.X, a.v.Y, a.v.Z);
+                // byte z + 3 of a code row is voxel z, the lane axis's first
+                // voxel z = 1 (codes along z: up to the end of the row's last
+                // word, zeros past Z)
+                const size_t oc = in ? (size_t)(x + 1) * a.cX + (size_t)(r + 1) * a.cR + (a.cL == 1 ? 4 : a.cL + 3) : 0;
+                const uint32_t nc = a.cL == 1 ? (uint32_t)a.cR - 4u : (uint32_t)((a.lane_n - 1) * a.cL + 1);
+                const rsrc_t rC = make_rsrc(C + oc, in ? nc : 0u);
+                const int vc = l0 * a.cL;
+                if (a.cL == 1 && P == 2) {
+                    K[row / 2] |= (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(rC, vc, 0, 0) << (16 * (row % 2));
+                } else if (a.cL == 1) {
 #pragma unroll
-                for (int e = 0; e < P; ++e) F[row][e] = ld_f32(rF, vo, e * a.sL * 4);
-            }
-            if (a.cL == 1 && P == 2) {
-                K[row / 2] |= (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(rC, vc, 0, 0) << (16 * (row % 2));
-            } else if (a.cL == 1) {
+                    for (int e = 0; e + 3 < P; e += 4)
+                        K[(row * P + e) / 4] = __builtin_amdgcn_raw_buffer_load_b32(rC, vc + e, 0, 0);
+                } else {
 #pragma unroll
-                for (int e = 0; e + 3 < P; e += 4)
-                    K[(row * P + e) / 4] = __builtin_amdgcn_raw_buffer_load_b32(rC, vc + e, 0, 0);
-            } else {
-#pragma unroll
-                for (int e = 0; e < P; ++e)
-                    K[(row * P + e) / 4] |= ld_u8(rC, vc, e * a.cL) << (8 * ((row * P + e) % 4));
+                    for (int e = 0; e < P; ++e)
+                        K[(row * P + e) / 4] |= ld_u8(rC, vc, e * a.cL) << (8 * ((row * P + e) % 4));
+                }
             }
         }
     }
@@ -255,26 +298,37 @@ __global__ __launch_bounds__(NW * 64) void k_resident(ResidentArgs a) {
         row_side(gy + 1, srp, wrp, Trp);
     }
     const int RYt = WY * PY, RXt = WX * PX, tile_rows = 2 * (RYt + RXt);
-    const size_t slot = (size_t)tile_rows * ROW;
     typedef unsigned long long word_t;
+    // mailbox places in bytes (the plan keeps it below 2 GiB): a row's words
+    // of slot 0; the other slot is `slot` bytes on
+    const uint32_t slot = (uint32_t)tile_rows * (ROW * 8);
     // place of a row among a tile's face rows: sides x-, x+, row-, row+
     auto face_row = [&](int side, int row) {
         return (side == 0 ? 0 : side == 1 ? RYt : side == 2 ? 2 * RYt : 2 * RYt + RXt) + row;
     };
-    auto box = [&](int tile, int side, int row) {  // a row's words of slot 0
-        return a.mail + ((size_t)tile * 2 * slot + (size_t)face_row(side, row) * ROW);
+    auto box = [&](int tile, int side, int row) {
+        return (uint32_t)tile * (2 * slot) + (uint32_t)face_row(side, row) * (ROW * 8);
     };
-    word_t* const in_x = box(T, sxm == kMail ? 0 : 1, wy * PY);
-    word_t* const in_r = box(T, srm == kMail ? 2 : 3, wx * PX);
+    const uint32_t in_x = box(T, sxm == kMail ? 0 : 1, wy * PY);
+    const uint32_t in_r = box(T, srm == kMail ? 2 : 3, wx * PX);
+    const uint32_t out_xm = box(Txm, 1, wy * PY), out_xp = box(Txp, 0, wy * PY);
+    const uint32_t out_rm = box(Trm, 3, wx * PX), out_rp = box(Trp, 2, wx * PX);
+    // word i of this lane from a place
+    // (from `at`, this lane's 8 bytes of a row, made anew where it is used:
+    // otherwise every place keeps a register of its own through the loop)
+    auto lane_bytes = [&]() {
+        uint32_t v = (uint32_t)lane * 8u;
+        asm volatile("" : "+v"(v));
+        return v;
+    };
+    auto word_of = [&](uint32_t place, uint32_t at, int i) {
+        return reinterpret_cast<word_t*>(reinterpret_cast<char*>(a.mail) + (place + at)) + i * 64;
+    };
     // where the rows of a side that no wave of this workgroup publishes are kept
     float* const f_xm = faces + face_row(0, wy * PY) * ROW + lane;
     float* const f_xp = faces + face_row(1, wy * PY) * ROW + lane;
     float* const f_rm = faces + face_row(2, wx * PX) * ROW + lane;
     float* const f_rp = faces + face_row(3, wx * PX) * ROW + lane;
-    word_t* const out_xm = box(Txm, 1, wy * PY);
-    word_t* const out_xp = box(Txp, 0, wy * PY);
-    word_t* const out_rm = box(Trm, 3, wx * PX);
-    word_t* const out_rp = box(Trp, 2, wx * PX);
     const bool in_row = l0 < a.lane_n;  // the other lanes' words are not sent
     const bool mail_x = sxm == kMail || sxp == kMail, mail_r = srm == kMail || srp == kMail;
     // lane of the row's last voxel (periodic rows fill it: lane_n % P == 0)
@@ -301,14 +355,15 @@ __global__ __launch_bounds__(NW * 64) void k_resident(ResidentArgs a) {
     // the rows of the tile faces, tagged, into the other tiles' slot
     auto send = [&](auto q_c, uint32_t tag, int sl) {
         constexpr int Q = decltype(q_c)::value;
-        auto put = [&](word_t* p, int ix, int iy, int at) {
+        const uint32_t lane8 = lane_bytes();
+        auto put = [&](uint32_t place, int ix, int iy, int at) {
             const int row = ix * PY + iy, ae = (Q ^ ix ^ iy) & 1;
 #pragma unroll
             for (int k = 0; k < HP; ++k) {
                 // a copy: F itself would be allocated as half of the word
                 float val = F[row][2 * k + ae];
                 asm volatile("" : "+v"(val));
-                __hip_atomic_store(p + sl * slot + (at * HP + k) * 64 + (uint32_t)lane,
+                __hip_atomic_store(word_of(place + sl * slot, lane8, at * HP + k),
                                    (word_t)tag << 32 | __builtin_bit_cast(uint32_t, val), __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
             }
@@ -332,13 +387,23 @@ __global__ __launch_bounds__(NW * 64) void k_resident(ResidentArgs a) {
     const float kz = KIND == TF_KIND_ANISOTROPIC ? a.table[TF_ANISO_TABLE - 1] : 0.0f;
     // weights of the row axis and of the lane axis
     const float k_row = a.sL == 1 ? ky : kz, k_lane = a.sL == 1 ? kz : ky;
+    // face codes: bits of the row axis's and of the lane axis's face
+    const int sh_row = a.sL == 1 ? 6 : 12, sh_lane = a.sL == 1 ? 12 : 6;
 
     auto half = [&](auto q_c, int t) {
         constexpr int Q = decltype(q_c)::value;
         // the packed codes as if new in every half-sweep: the compiler would
         // otherwise keep every extracted byte in a register of its own
+        // (the field kind: the sums of the faces, where they would not fit)
+        if constexpr (kBytes) {
 #pragma unroll
-        for (int i = 0; i < NK; ++i) asm volatile("" : "+v"(K[i]));
+            for (int i = 0; i < NK; ++i) asm volatile("" : "+v"(K[i]));
+        } else if constexpr (kFaceCodes || E > 8) {
+#pragma unroll
+            for (int i = 0; i < R; ++i)
+#pragma unroll
+                for (int e = 0; e < P; ++e) asm volatile("" : "+v"(G[0][i][e]));
+        }
         // the x ghost plane xg next to row ix of the patch: constant
         auto ghost_x = [&](float* d, int xg, int ix) {
             const rsrc_t r = make_rsrc(S + (size_t)xg * a.v.sX, (uint32_t)a.v.sX * 4u);
@@ -360,7 +425,7 @@ __global__ __launch_bounds__(NW * 64) void k_resident(ResidentArgs a) {
             constexpr int NX = HX ? PY * HP : 0, N = NX + (HR ? PX * HP : 0);
             if (!in_row) return;
             const uint32_t tag = a.tag0 + (uint32_t)t;
-            const size_t so = (t & 1) * slot;
+            const uint32_t so = (t & 1) * slot, lane8 = lane_bytes();
             word_t m[N];
             for (int n = dead ? a.spin : 0;; ++n) {
                 // (no pause, and one question at a time: a first question 0.3
@@ -368,10 +433,9 @@ __global__ __launch_bounds__(NW * 64) void k_resident(ResidentArgs a) {
                 // cost 0.1 to 0.3 us per half-sweep from 32^3 to 200^3)
                 bool ok = true;
 #pragma unroll
-                for (int i = 0; i < N; ++i) {
-                    const word_t* const p = i < NX ? in_x + so + i * 64 : in_r + so + (i - NX) * 64;
-                    m[i] = __hip_atomic_load(p + (uint32_t)lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                }
+                for (int i = 0; i < N; ++i)
+                    m[i] = __hip_atomic_load(i < NX ? word_of(in_x + so, lane8, i) : word_of(in_r + so, lane8, i - NX),
+                                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
                 for (int i = 0; i < N; ++i) ok = ok && (uint32_t)(m[i] >> 32) == tag;
                 if (__builtin_amdgcn_ballot_w64(!ok) == 0) break;
@@ -437,38 +501,87 @@ __global__ __launch_bounds__(NW * 64) void k_resident(ResidentArgs a) {
                         lp = lane == last_lane ? wrapped : lp;
                     }
                 }
-                constexpr int at = row * P + e;
-                const uint32_t code = (K[at / 4] >> (8 * (at % 4))) & 0xffu;
-                const float2 rf = *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(rs_smem) +
-                                                                   (kPairs ? code * 8 : code));
-                float sum = xp + xm;
-                if constexpr (KIND == TF_KIND_ANISOTROPIC) {
-                    float u = rp + rm;
-                    u = k_row * u;
-                    sum = sum + u;
-                    u = lp + lm;
-                    u = k_lane * u;
-                    sum = sum + u;
+                if constexpr (kBytes) {
+                    constexpr int at = row * P + e;
+                    const uint32_t code = (K[at / 4] >> (8 * (at % 4))) & 0xffu;
+                    const float2 rf = *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(rs_smem) +
+                                                                       (kPairs ? code * 8 : code));
+                    float sum = xp + xm;
+                    if constexpr (KIND == TF_KIND_ANISOTROPIC) {
+                        float u = rp + rm;
+                        u = k_row * u;
+                        sum = sum + u;
+                        u = lp + lm;
+                        u = k_lane * u;
+                        sum = sum + u;
+                    } else {
+                        sum = sum + rp;
+                        sum = sum + rm;
+                        sum = sum + lp;
+                        sum = sum + lm;
+                    }
+                    s[j] = sum;
+                    f[j] = rf.y;
+                    q[j] = sum * rf.x;
+                    const float res = __builtin_fmaf(-q[j], rf.y, sum);
+                    q[j] = __builtin_fmaf(res, rf.x, q[j]);
+                    // the reciprocal is not exact: a subnormal residual
+                    // (Solver), a tiny sum, or nothing finite (prefactor_pair)
+                    rare = rare || (kPairs ? __builtin_amdgcn_frexp_expf(sum) < rare_below ||
+                                                 __builtin_amdgcn_classf(res, 0x207)
+                                           : __builtin_amdgcn_classf(res, 0x90));
                 } else {
-                    sum = sum + rp;
-                    sum = sum + rm;
-                    sum = sum + lp;
-                    sum = sum + lm;
+                    // the six faces: the voxel's own plus faces and those of
+                    // its neighbours on the minus sides
+                    auto word = [](float w) { return __builtin_bit_cast(uint32_t, w); };
+                    float wxm, wrm, wlm;
+                    if constexpr (ix > 0) wxm = G[0][row - PY][e]; else wxm = Gx[iy][e];
+                    if constexpr (iy > 0) wrm = G[kField ? 1 : 0][row - 1][e]; else wrm = Gr[ix][e];
+                    if constexpr (e > 0) wlm = G[kField ? 2 : 0][row][e - 1]; else wlm = Gl[row];
+                    float gxp, gxm, grp, grm, glp, glm;
+                    if constexpr (kField) {
+                        gxp = G[0][row][e], grp = G[1][row][e], glp = G[2][row][e];
+                        gxm = wxm, grm = wrm, glm = wlm;
+                    } else {
+                        const char* const tb = reinterpret_cast<const char*>(rs_smem);
+                        auto face = [tb](uint32_t c, int at) {
+                            return *reinterpret_cast<const float*>(tb + ((c >> at) & 63u));
+                        };
+                        const uint32_t own = word(G[0][row][e]);
+                        gxp = face(own, 0), grp = face(own, sh_row), glp = face(own, sh_lane);
+                        gxm = face(word(wxm), 0), grm = face(word(wrm), sh_row), glm = face(word(wlm), sh_lane);
+                    }
+                    float sum = xp * gxp + xm * gxm;
+                    sum = sum + rp * grp;
+                    sum = sum + rm * grm;
+                    sum = sum + lp * glp;
+                    sum = sum + lm * glm;
+                    if constexpr (kField) {
+                        float fs = gxm + gxp;
+                        fs = fs + grm;
+                        fs = fs + grp;
+                        fs = fs + glm;
+                        fs = fs + glp;
+                        // fma with a factor 0 or 1 rounds as the sum
+                        if constexpr (ix == 0) fs = __builtin_fmaf(gxm, first, fs);
+                        fs = __builtin_fmaf(gxp, last[ix], fs);
+                        if (fs == 0.0f) fs = __builtin_inff();
+                        q[j] = sum / fs;
+                    } else {
+                        const float2 rf = *reinterpret_cast<const float2*>(
+                            reinterpret_cast<const char*>(rs_smem) + 4 * TF_MPF_FACE_SLOTS + (word(G[0][row][e]) >> 18));
+                        s[j] = sum;
+                        f[j] = rf.y;
+                        q[j] = sum * rf.x;
+                        const float res = __builtin_fmaf(-q[j], rf.y, sum);
+                        q[j] = __builtin_fmaf(res, rf.x, q[j]);
+                        rare = rare || __builtin_amdgcn_frexp_expf(sum) < -99;  // as rsweep_tile
+                    }
                 }
-                s[j] = sum;
-                f[j] = rf.y;
-                q[j] = sum * rf.x;
-                const float res = __builtin_fmaf(-q[j], rf.y, sum);
-                q[j] = __builtin_fmaf(res, rf.x, q[j]);
-                // the reciprocal is not exact: a subnormal residual (Solver),
-                // a tiny sum, or nothing finite (prefactor_pair)
-                rare = rare || (kPairs ? __builtin_amdgcn_frexp_expf(sum) < rare_below ||
-                                             __builtin_amdgcn_classf(res, 0x207)
-                                       : __builtin_amdgcn_classf(res, 0x90));
             });
             // those quotients are divided; the pair (0, 0) stands for an
             // infinite prefactor
-            if (__builtin_expect(__builtin_amdgcn_ballot_w64(rare) != 0, 0)) {
+            if (!kField && __builtin_expect(__builtin_amdgcn_ballot_w64(rare) != 0, 0)) {
 #pragma unroll
                 for (int j = 0; j < N; ++j) q[j] = f[j] != 0.0f ? s[j] / f[j] : s[j] / __builtin_inff();
             }
@@ -480,13 +593,14 @@ __global__ __launch_bounds__(NW * 64) void k_resident(ResidentArgs a) {
                 d = d * wrow[ix];
                 F[row][e] = c + d;
             });
+            if constexpr (kField) __builtin_amdgcn_sched_barrier(0);
         };
         auto update_all = [&](auto from_c, auto to_c) {
             constexpr int from = decltype(from_c)::value, to = decltype(to_c)::value;
-            constexpr int G = E <= 32 || E > 64 ? 4 : 8;  // quotients per test
-            static_for<0, (to - from + G - 1) / G>([&](auto g_c) {
-                constexpr int i = from + decltype(g_c)::value * G;
-                update(ic<i>{}, ic<(to - i < G ? to - i : G)>{});
+            constexpr int M = kFaceCodes || (kField && E > 32) ? 2 : !kBytes || E <= 32 || E > 64 ? 4 : 8;  // quotients per test
+            static_for<0, (to - from + M - 1) / M>([&](auto g_c) {
+                constexpr int i = from + decltype(g_c)::value * M;
+                update(ic<i>{}, ic<(to - i < M ? to - i : M)>{});
             });
         };
         // the border rows first: their messages are on the way while the
@@ -587,11 +701,29 @@ static int launch_resident(const ResidentArgs& a, hipStream_t st) {
     F(8, 1, 1, 16) F(8, 1, 2, 16) F(8, 2, 2, 16) F(8, 2, 3, 8) F(8, 3, 4, 8) \
     F(16, 1, 1, 16) F(16, 2, 2, 8) F(32, 1, 1, 8)
 
+// Face codes take a word per voxel: half the voxels per register.
+#define TF_RESIDENT_SHAPES_FACES(F) \
+    F(2, 1, 1, 16) F(2, 1, 2, 16) F(2, 2, 2, 16) F(2, 2, 4, 16) F(2, 4, 6, 8) \
+    F(4, 1, 1, 16) F(4, 1, 2, 16) F(4, 2, 2, 16) F(4, 3, 3, 8) F(4, 3, 4, 8) \
+    F(8, 1, 1, 16) F(8, 1, 2, 16) F(8, 2, 3, 8) F(16, 1, 1, 8) F(16, 1, 2, 8)
+
+// The field kind takes three words per voxel.
+#define TF_RESIDENT_SHAPES_FIELD(F) \
+    F(2, 1, 1, 16) F(2, 1, 2, 16) F(2, 2, 2, 16) F(2, 2, 3, 16) F(2, 4, 4, 8) \
+    F(4, 1, 1, 16) F(4, 1, 2, 16) F(4, 1, 3, 16) F(4, 2, 4, 8) F(4, 3, 3, 8) \
+    F(8, 1, 1, 16) F(8, 1, 3, 8) F(8, 2, 2, 8) F(16, 1, 1, 8)
+
 template <int KIND, bool PER>
 static int dispatch_resident(const tf_resident& p, const ResidentArgs& a, hipStream_t st) {
 #define F(P, PX, PY, NW) \
     if (p.elems == P && p.px == PX && p.py == PY && p.waves == NW) return launch_resident<KIND, P, PX, PY, NW, PER>(a, st);
-    TF_RESIDENT_SHAPES(F)
+    if constexpr (KIND == TF_KIND_FIELD) {
+        TF_RESIDENT_SHAPES_FIELD(F)
+    } else if constexpr (KIND == TF_KIND_MULTIPHASE_FACES) {
+        TF_RESIDENT_SHAPES_FACES(F)
+    } else {
+        TF_RESIDENT_SHAPES(F)
+    }
 #undef F
     return fail(-1, "resident shape (%d, %d, %d, %d) is not compiled", p.elems, p.px, p.py, p.waves);
 }
@@ -601,3 +733,5 @@ int resident_dispatch_solver(const tf_resident& p, const ResidentArgs& a, hipStr
 int resident_dispatch_periodic(const tf_resident& p, const ResidentArgs& a, hipStream_t st);
 int resident_dispatch_anisotropic(const tf_resident& p, const ResidentArgs& a, hipStream_t st);
 int resident_dispatch_electrode(const tf_resident& p, const ResidentArgs& a, int periodic, hipStream_t st);
+int resident_dispatch_field(const tf_resident& p, const ResidentArgs& a, hipStream_t st);
+int resident_dispatch_mpfaces(const tf_resident& p, const ResidentArgs& a, hipStream_t st);

@@ -408,6 +408,18 @@ class SORSolver(ABC):
             self._resident = _ResidentSweep.make(self) or False
         return bool(self._resident)
 
+    def _resident_kind(self):
+        """Kind (with the sweep flags) of this solver's resident sweep, None
+        if it has none."""
+        if self.kind in (_lib.KIND_SOLVER, _lib.KIND_ANISOTROPIC, _lib.KIND_ELECTRODE, _lib.KIND_FIELD):
+            return self.kind | self._sweep_flags
+        return None
+
+    def _resident_operands(self):
+        """(codes, table, table length) the resident sweep reads."""
+        _, codes, table, n_table = self._sweep_target()
+        return codes, table, n_table
+
     def _settle(self) -> None:
         """Make sure that the resident launches since the last check ran to
         their end (waits for them); repeat them otherwise."""
@@ -607,21 +619,32 @@ class _ResidentSweep:
 
     @classmethod
     def make(cls, s):
-        kind = s.kind | s._sweep_flags
-        if s.kind not in (_lib.KIND_SOLVER, _lib.KIND_ANISOTROPIC, _lib.KIND_ELECTRODE):
+        kind = s._resident_kind()
+        if kind is None:
             return None
         plan = _lib.Resident()
         cus = torch.cuda.get_device_properties(s.device).multi_processor_count
-        r = s._lib.tf_resident_plan(kind, s.batch_size, s.Nx, s.Ny, s.Nz, cus, ctypes.byref(plan))
-        if r < 0:
-            _lib.check(r, "tf_resident_plan")
-        return cls(s, kind, plan) if r else None
+        # the kinds with face conductances also run batches in several
+        # launches (groups of equally many volumes): 0.7 ns per voxel and
+        # half-sweep of 4 x 128^3 against 1.6 streaming; the others stream a
+        # batch that does not fit at once, at 0.5 to 0.7 ns
+        B = s.batch_size
+        most = B if kind in (_lib.KIND_FIELD, _lib.KIND_MULTIPHASE_FACES) else 1
+        for groups in range(1, most + 1):
+            per = -(-B // groups)
+            r = s._lib.tf_resident_plan(kind, per, s.Nx, s.Ny, s.Nz, cus, ctypes.byref(plan))
+            if r < 0:
+                _lib.check(r, "tf_resident_plan")
+            if r:
+                return cls(s, kind, per, plan)
+        return None
 
-    def __init__(self, s, kind, plan):
-        self.kind, self.plan = kind, plan
+    def __init__(self, s, kind, per, plan):
+        self.kind, self.per, self.plan = kind, per, plan
+        self.codes, self.table, self.n_table = s._resident_operands()
         self.mail = torch.zeros(plan.mail_bytes // 8, dtype=torch.int64, device=s.device)
         self.status = s._sums[-1:].view(torch.int32)[:1]
-        self.third = None  # see _PeriodicYZ._advance
+        self.third = None  # see _PeriodicYZ._last_half_sweep
         self.spin = 0
         self.tag, self.count = 1, 0
         self.log = []  # (number, field read, first iteration) of each launch
@@ -629,25 +652,32 @@ class _ResidentSweep:
     def launch(self, s, n: int, it: int) -> bool:
         """n half-sweeps from iteration it; False if the device does not hold
         the workgroups (the solver streams from then on)."""
-        if self.tag + n + 1 >= 2 ** 32:
-            self.mail.zero_()
-            self.tag = 1
+        B, X, Y, Z = s.batch_size, s.Nx, s.Ny, s.Nz
         src, dst = s._fields[s._cur], s._fields[1 - s._cur]
         self.count += 1
-        _, codes, table, _ = s._sweep_pointers()
         ev = s._launch_events
         if ev is not None:
             t0, t1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
             t0.record()
         stream = torch.cuda.current_stream(s.device)
+        volume = 4 * (X + 2) * (Y + 2) * (Z + 2)  # bytes of a field (and of face words)
+        table = _lib.ptr(self.table) if self.table is not None else None
         with _resident_lock:
             last = _resident_turn.get(s.device.index)
             if last is not None and last != stream:
                 stream.wait_event(last.record_event())
-            st = s._lib.tf_sweep_resident(_lib.ptr(src), _lib.ptr(dst), codes, table, self.kind, s.batch_size, s.Nx,
-                                          s.Ny, s.Nz, s._w32, it & 1, n, self.plan, _lib.ptr(self.mail),
-                                          self.plan.mail_bytes, self.tag, _lib.ptr(self.status), self.count,
-                                          self.spin, stream.cuda_stream)
+            for b in range(0, B, self.per):
+                if self.tag + n + 1 >= 2 ** 32:
+                    self.mail.zero_()
+                    self.tag = 1
+                st = s._lib.tf_sweep_resident(_lib.ptr(src) + b * volume, _lib.ptr(dst) + b * volume,
+                                              _lib.ptr(self.codes) + b * volume, table, self.n_table, self.kind,
+                                              min(self.per, B - b), X, Y, Z, s._w32, it & 1, n, self.plan,
+                                              B * volume // 4, _lib.ptr(self.mail), self.plan.mail_bytes, self.tag,
+                                              _lib.ptr(self.status), self.count, self.spin, stream.cuda_stream)
+                if st != 0:
+                    break
+                self.tag += n + 1
             _resident_turn[s.device.index] = stream
         if st == _lib.NOT_RESIDENT and not self.log:
             s._resident = False
@@ -656,7 +686,6 @@ class _ResidentSweep:
         if ev is not None:
             t1.record()
             ev.append((t0, t1, 1))
-        self.tag += n + 1
         self.log.append((self.count, src, it))
         s._cur = 1 - s._cur
         return True
@@ -1150,6 +1179,24 @@ class MultiPhaseSolver(ThroughTransportSolver):
             return super()._sweep_target()
         t = self._faces["table"]
         return _lib.KIND_MULTIPHASE_FACES, self._faces["codes"], t, t.numel()
+
+    def _resident_kind(self):
+        if self._sweep_flags:
+            return None  # periodic y/z
+        if self._faces is not None:
+            return _lib.KIND_MULTIPHASE_FACES if self._faces["table"].numel() <= _lib.RESIDENT_TABLE else None
+        # class codes sweep through the face conductances of their classes
+        return _lib.KIND_FIELD
+
+    def _resident_operands(self):
+        if self._faces is not None or self._field_faces is not None:
+            return super()._resident_operands()
+        B, X, Y, Z = self.batch_size, self.Nx, self.Ny, self.Nz
+        faces = _lib.slack_buffer((3, B, X + 2, Y + 2, Z + 2), torch.float32, self.device)
+        st = self._lib.tf_class_faces(_lib.ptr(self._codes), _lib.ptr(self._hm_lut), self._n_classes,
+                                      _lib.ptr(faces), B, X, Y, Z, self._stream())
+        _lib.check(st, "tf_class_faces")
+        return faces, None, 0
 
     def _class_image(self, labels, cls_of_label) -> np.ndarray:
         img = self.cpu_img

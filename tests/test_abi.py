@@ -145,7 +145,8 @@ def test_resident_plan():
     assert plan(0, 1, 8, 8, 2100) == 0  # longer than 64 lanes of 32 voxels
     assert plan(_lib.SWEEP_PERIODIC_YZ, 1, 20, 20, 130) == 0  # a wrapped row must end with its lane
     assert plan(_lib.KIND_MULTIPHASE, 1, 8, 8, 8) < 0 and plan(0, 0, 8, 8, 8) < 0
-    assert lib.tf_sweep_resident(1, 1, 1, None, 0, 1, 4, 4, 4, 1.5, 0, 2, p, 1, 8, 1, 1, 1, 0, None) < 0
+    assert lib.tf_sweep_resident(1, 1, 1, None, 0, 0, 1, 4, 4, 4, 1.5, 0, 2, p, 0, 1, 8, 1, 1, 1, 0, None) < 0
     assert plan(0, 1, 40, 40, 40) == 1
-    st = lib.tf_sweep_resident(4, 8, 1, None, 0, 1, 40, 40, 40, 1.5, 0, 2, p, 8, p.mail_bytes - 8, 1, 1, 1, 0, None)
+    st = lib.tf_sweep_resident(4, 8, 1, None, 0, 0, 1, 40, 40, 40, 1.5, 0, 2, p, 0, 8, p.mail_bytes - 8, 1, 1, 1, 0,
+                               None)
     assert st < 0 and b"mailbox" in lib.tf_last_error()

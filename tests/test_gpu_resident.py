@@ -8,8 +8,8 @@ import pytest
 import torch
 
 import taufactor_amd as tau
-from oracle.restate import (OracleAnisotropicSolver, OracleElectrodeSolver, OraclePeriodicElectrodeSolver,
-                            OraclePeriodicSolver, OracleSolver)
+from oracle.restate import (OracleAnisotropicSolver, OracleElectrodeSolver, OracleFieldSolver, OracleMultiPhaseSolver,
+                            OraclePeriodicElectrodeSolver, OraclePeriodicSolver, OracleSolver)
 
 pytestmark = pytest.mark.gpu
 
@@ -142,3 +142,77 @@ def test_streams_take_turns():
     for s, img in zip(solvers, imgs):
         assert s._resident
         assert np.array_equal(s.field.cpu().numpy(), OracleSolver(img).run(310).field.numpy())
+
+
+def _map(shape, seed):
+    """Voxel diffusivities, a fifth of them 0."""
+    rng = np.random.default_rng(seed)
+    k = rng.uniform(0.05, 2.0, size=shape).astype(np.float32)
+    k[rng.random(shape) < 0.2] = 0.0
+    return k
+
+
+@pytest.mark.parametrize("shape,plan", [
+    ((3, 4, 5), (2, 1, 1, 16)), ((9, 8, 127), (2, 1, 1, 16)), ((100, 60, 5), (2, 1, 2, 16)),
+    ((120, 72, 5), (2, 2, 2, 16)), ((130, 130, 5), (2, 2, 3, 16)), ((215, 129, 5), (2, 4, 4, 8)),
+    ((7, 5, 140), (4, 1, 1, 16)), ((100, 60, 140), (4, 1, 2, 16)), ((120, 72, 140), (4, 1, 3, 16)),
+    ((150, 90, 140), (4, 2, 4, 8)), ((130, 130, 140), (4, 3, 3, 8)), ((6, 3, 260), (8, 1, 1, 16)),
+    ((100, 60, 260), (8, 1, 3, 8)), ((80, 80, 260), (8, 2, 2, 8)), ((6, 3, 520), (16, 1, 1, 8))])
+def test_field_every_patch(shape, plan):
+    k = _map(shape, 2)
+    s = tau.FieldSolver(k)
+    assert s._resident_sweep()
+    p = s._resident.plan
+    assert (p.elems, p.px, p.py, p.waves) == plan
+    _same(s, OracleFieldSolver(k), 7)
+
+
+def test_field_batch_in_groups():
+    """Five volumes of which two fit at once, checks and a resumed solve."""
+    k = _map((5, 112, 100, 90), 3)
+    s = tau.FieldSolver(k)
+    assert s._resident_sweep() and 1 < s._resident.per < 5
+    _same(s, OracleFieldSolver(k), 103)
+
+
+def _labels(shape, n, seed):
+    return np.random.default_rng(seed).integers(0, n, size=shape).astype(np.uint8)
+
+
+D3 = {0: 0.0, 1: 1.0, 2: 0.1}
+D7 = {0: 0.0, 1: 1.0, 2: 0.5, 3: 0.25, 4: 0.12, 5: 2.0, 6: 1 / 3}
+
+
+@pytest.mark.parametrize("shape,plan", [
+    ((3, 4, 5), (2, 1, 1, 16)), ((9, 8, 127), (2, 1, 1, 16)), ((100, 60, 5), (2, 1, 2, 16)),
+    ((120, 72, 5), (2, 2, 2, 16)), ((130, 130, 5), (2, 2, 4, 16)), ((230, 138, 5), (2, 4, 6, 8)),
+    ((7, 5, 140), (4, 1, 1, 16)), ((100, 60, 140), (4, 1, 2, 16)), ((120, 72, 140), (4, 2, 2, 16)),
+    ((130, 130, 140), (4, 3, 3, 8)), ((185, 111, 140), (4, 3, 4, 8)), ((6, 3, 260), (8, 1, 1, 16)),
+    ((100, 60, 260), (8, 1, 2, 16)), ((120, 72, 260), (8, 2, 3, 8)), ((6, 3, 520), (16, 1, 1, 8)),
+    ((60, 36, 520), (16, 1, 2, 8))])
+def test_multiphase_every_patch(shape, plan):
+    img = _labels(shape, 3, 7)
+    s = tau.MultiPhaseSolver(img, dict(D3))
+    assert s._resident_sweep()
+    p = s._resident.plan
+    assert (p.elems, p.px, p.py, p.waves) == plan
+    _same(s, OracleMultiPhaseSolver(img, dict(D3)), 7)
+
+
+@pytest.mark.parametrize("Ds,n", [(D3, 3), (D7, 7)])
+@pytest.mark.parametrize("shape", [(14, 13, 12), (8, 9, 131), (33, 150), (2, 9, 8, 70)])
+def test_multiphase_blocks(Ds, n, shape):
+    """Face codes and (seven values) class codes over two blocks, first and
+    last layers, images and batches."""
+    img = _labels(shape, n, 11)
+    _same(tau.MultiPhaseSolver(img, dict(Ds)), OracleMultiPhaseSolver(img, dict(Ds)), 109)
+
+
+def test_field_and_multiphase_lost_waits():
+    k, img = _map((3, 60, 61, 62), 4), _labels((50, 51, 52), 3, 5)
+    for s, o in ((tau.FieldSolver(k), OracleFieldSolver(k)),
+                 (tau.MultiPhaseSolver(img, dict(D3)), OracleMultiPhaseSolver(img, dict(D3)))):
+        assert s._resident_sweep()
+        s._resident.spin = 1
+        s.solve(iter_limit=130, verbose=False, conv_crit=0.0)
+        assert np.array_equal(s.field.cpu().numpy(), o.run(130).field.numpy())
