@@ -597,7 +597,7 @@ extern "C" int tf_sweep_launch_config(int kind, int n_classes, int B, int X, int
 // ---------------------------------------------------------------------------
 struct ResidentShapeDesc {
     int elems, px, py, waves;
-    size_t (*lds_floats)(int wy);  // (code kinds: with the largest table)
+    size_t (*lds_floats)(int wy);
 };
 template <int KIND>
 static const std::vector<ResidentShapeDesc>& resident_shapes_of() {
@@ -608,8 +608,11 @@ static const std::vector<ResidentShapeDesc>& resident_shapes_of() {
     } else if constexpr (KIND == TF_KIND_MULTIPHASE_FACES) {
         static const std::vector<ResidentShapeDesc> v = {TF_RESIDENT_SHAPES_FACES(F)};
         return v;
-    } else {
+    } else if constexpr (KIND == TF_KIND_SOLVER) {
         static const std::vector<ResidentShapeDesc> v = {TF_RESIDENT_SHAPES(F)};
+        return v;
+    } else {
+        static const std::vector<ResidentShapeDesc> v = {TF_RESIDENT_SHAPES_PAIRS(F)};
         return v;
     }
 #undef F
@@ -617,6 +620,7 @@ static const std::vector<ResidentShapeDesc>& resident_shapes_of() {
 static const std::vector<ResidentShapeDesc>& resident_shapes(int kind) {
     return kind == TF_KIND_FIELD               ? resident_shapes_of<TF_KIND_FIELD>()
            : kind == TF_KIND_MULTIPHASE_FACES ? resident_shapes_of<TF_KIND_MULTIPHASE_FACES>()
+           : kind == TF_KIND_SOLVER           ? resident_shapes_of<TF_KIND_SOLVER>()
                                               : resident_shapes_of<TF_KIND_ANISOTROPIC>();
 }
 

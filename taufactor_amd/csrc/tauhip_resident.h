@@ -9,9 +9,12 @@
 // registers for the whole launch, so a half-sweep moves only tile faces, and
 // no voxel is updated twice.  Per half-sweep, streaming and resident, on
 // MI355X (256 compute units):
-//   32^3 2.9, 1.3 us; 100^3 3.3, 1.5; 128^3 3.7, 1.7; 160^3 5.3, 3.1;
-//   203 x 157 x 181 7.4, 4.3; 200^3 7.8, 5.0; 611 x 803 pixels 18, 1.8;
-//   1500 x 1600 pixels 60, 2.4
+//   32^3 2.9, 1.2 us; 100^3 3.3, 1.5; 128^3 3.7, 1.7; 160^3 5.4, 3.2;
+//   203 x 157 x 181 7.4, 4.3; 200^3 7.8, 4.6; 220^3 7.1, 5.8;
+//   256^3 11.3, 6.2; 611 x 803 pixels 18, 1.8; 1500 x 1600 60, 2.5;
+//   per-voxel field 128^3 6.4, 1.8, two of them 10, 2.9;
+//   three-phase 128^3 5.5, 2.0, 160^3 8.0, 5.5; seven values
+//   121 x 130 x 143 10.1, 4.4
 // Bound: up to 128^3 the exchange of the faces (without it 0.4 to 0.8 us),
 // beyond it issue and the exchange about evenly (200^3: 3.5 us without it).
 //
@@ -28,8 +31,7 @@
 // counts half-sweeps across launches, written and read with relaxed
 // device-scope atomics, so no flag, fence or second round trip follows the
 // data: 1.0 to 1.3 us from the update of a border row to its use in another
-// workgroup.  Two slots per row suffice: a
-// wave sends half-sweep t + 1's rows after it has read its partner's of t,
+// workgroup.  Two slots per row suffice: a wave sends half-sweep t + 1's rows after it has read its partner's of t,
 // which the partner sent after reading the slot that is written again.
 //
 // Progress.  The workgroups wait for each other, so all of them have to be
@@ -81,6 +83,7 @@ struct ResidentShape {
     static constexpr int HP = P / 2;            // voxels of one colour per lane and row
     static constexpr int E = R * P;             // voxels per lane
     static constexpr int ROW = HP * 64;         // floats of one colour of a row
+    static constexpr bool kEven = PX % 2 == 0 && PY % 2 == 0;
     static constexpr int inner(int p) { return p > 2 ? p - 2 : 0; }
     static constexpr int RB = R - inner(PX) * inner(PY);  // border rows of a patch
     static constexpr bool border(int row) {
@@ -119,7 +122,8 @@ struct ResidentShape {
     static constexpr size_t lds_floats(int wy) { return (size_t)HEAD + NBUF * PUB + face(wy) + ZERO; }
 };
 
-template <int KIND, int P, int PX, int PY, int NW, bool PER>
+// Q0: the launch's first colour where the patch has even sides, else 0
+template <int KIND, int P, int PX, int PY, int NW, bool PER, int Q0>
 __global__ __launch_bounds__(NW * 64) void k_resident(ResidentArgs a) {
     using Sh = ResidentShape<KIND, P, PX, PY, NW>;
     constexpr int R = Sh::R, RB = Sh::RB, HP = Sh::HP, E = Sh::E, ROW = Sh::ROW, NBUF = Sh::NBUF, PUB = Sh::PUB;
@@ -336,7 +340,7 @@ __global__ __launch_bounds__(NW * 64) void k_resident(ResidentArgs a) {
 
     // colour of the patch's first voxel: element e of row (ix, iy) is updated
     // in half-sweep t when e = Q ^ ix ^ iy (mod 2), Q = q0 ^ t (mod 2)
-    const int q0 = (a.colour0 ^ (gx * PX) ^ (gy * PY)) & 1;
+    const int q0 = Sh::kEven ? Q0 : (a.colour0 ^ (gx * PX) ^ (gy * PY)) & 1;
     bool dead = false;
     __syncthreads();
     const int rare_below = kPairs && s_flag[1] != 0 ? 1024 : -99;
@@ -621,6 +625,24 @@ __global__ __launch_bounds__(NW * 64) void k_resident(ResidentArgs a) {
         }
     }
     __syncthreads();
+    // one half-sweep and what it publishes; the barriers are the workgroup's
+    auto step = [&](auto q_c, int t) {
+        if (live) half(q_c, t);
+        if constexpr (NBUF == 1) __syncthreads();  // the edges have been read
+        if (live) publish(q_c, NBUF == 2 ? t & 1 : 0);
+        __syncthreads();
+    };
+    if constexpr (Sh::kEven) {
+        // every patch starts on the same colour, the kernel's own Q0: the two
+        // colours' half-sweeps in a row, without a branch whose sides would
+        // join the whole patch in other registers (128 voxels per lane: 74
+        // registers spilled with it, none without)
+        for (int t = 0; t < a.n_half; t += 2) {
+            step(ic<Q0>{}, t);
+            if (t + 1 == a.n_half) break;
+            step(ic<Q0 ^ 1>{}, t + 1);
+        }
+    } else {
     for (int t = 0; t < a.n_half; ++t) {
         const bool odd = ((q0 ^ t) & 1) != 0;
         if constexpr (NBUF == 2) {
@@ -647,6 +669,8 @@ __global__ __launch_bounds__(NW * 64) void k_resident(ResidentArgs a) {
         __syncthreads();
     }
 
+    }
+
     if (!live) return;
     float* const D = a.dst + (size_t)b * a.v.sB;
 #pragma unroll
@@ -666,10 +690,10 @@ __global__ __launch_bounds__(NW * 64) void k_resident(ResidentArgs a) {
         }
 }
 
-template <int KIND, int P, int PX, int PY, int NW, bool PER>
-static int launch_resident(const ResidentArgs& a, hipStream_t st) {
+template <int KIND, int P, int PX, int PY, int NW, bool PER, int Q0>
+static int launch_resident_colour(const ResidentArgs& a, hipStream_t st) {
     using Sh = ResidentShape<KIND, P, PX, PY, NW>;
-    const auto fn = k_resident<KIND, P, PX, PY, NW, PER>;
+    const auto fn = k_resident<KIND, P, PX, PY, NW, PER, Q0>;
     const size_t lds = Sh::lds_floats(a.WY) * sizeof(float);
     if (lds > 160 * 1024) return fail(TF_NOT_RESIDENT, "a resident tile needs %zu B of LDS", lds);
     static bool attr_set = false;
@@ -689,23 +713,33 @@ static int launch_resident(const ResidentArgs& a, hipStream_t st) {
     return 0;
 }
 
-// The compiled shapes, those that some volume's plan takes: (voxels per lane and row, patch rows in x, patch rows
-// of the other axis, waves).  Up to 32 voxels per lane the workgroup has 16
-// waves (128 registers per lane); larger patches need 8 (256 registers).  96
-// voxels per lane are the most that pay: with 128, for which some registers
-// spill, a half-sweep of 220^3 takes 8.1 us and of 256^3 11.3, the streaming
-// sweep's 7.1 and 11.3.
-#define TF_RESIDENT_SHAPES(F) \
+template <int KIND, int P, int PX, int PY, int NW, bool PER>
+static int launch_resident(const ResidentArgs& a, hipStream_t st) {
+    if constexpr (ResidentShape<KIND, P, PX, PY, NW>::kEven)
+        if (a.colour0) return launch_resident_colour<KIND, P, PX, PY, NW, PER, 1>(a, st);
+    return launch_resident_colour<KIND, P, PX, PY, NW, PER, 0>(a, st);
+}
+
+// The compiled shapes, those that some volume's plan takes: (voxels per lane
+// and row, patch rows in x, patch rows of the other axis, waves).  Up to 32
+// voxels per lane the workgroup has 16 waves (128 registers per lane); larger
+// patches need 8 (256 registers).  No loop spills more than a few registers:
+// a reload waits for every store before it, so one between the sends waits a
+// microsecond for their acknowledgement.  That bounds each kind's patches.
+#define TF_RESIDENT_SHAPES_PAIRS(F) \
     F(2, 1, 1, 16) F(2, 1, 2, 16) F(2, 2, 2, 16) F(2, 2, 4, 16) F(2, 4, 4, 16) F(2, 6, 8, 8) \
-    F(4, 1, 1, 16) F(4, 1, 2, 16) F(4, 2, 2, 16) F(4, 2, 3, 16) F(4, 2, 4, 16) F(4, 4, 5, 8) F(4, 4, 6, 8) \
+    F(4, 1, 1, 16) F(4, 1, 2, 16) F(4, 2, 2, 16) F(4, 2, 3, 16) F(4, 2, 4, 16) F(4, 4, 6, 8) \
     F(8, 1, 1, 16) F(8, 1, 2, 16) F(8, 2, 2, 16) F(8, 2, 3, 8) F(8, 3, 4, 8) \
     F(16, 1, 1, 16) F(16, 2, 2, 8) F(32, 1, 1, 8)
 
+// the Solver kind: 128 voxels per lane as well
+#define TF_RESIDENT_SHAPES(F) TF_RESIDENT_SHAPES_PAIRS(F) F(2, 8, 8, 8) F(4, 4, 8, 8)
+
 // Face codes take a word per voxel: half the voxels per register.
 #define TF_RESIDENT_SHAPES_FACES(F) \
-    F(2, 1, 1, 16) F(2, 1, 2, 16) F(2, 2, 2, 16) F(2, 2, 4, 16) F(2, 4, 6, 8) \
-    F(4, 1, 1, 16) F(4, 1, 2, 16) F(4, 2, 2, 16) F(4, 3, 3, 8) F(4, 3, 4, 8) \
-    F(8, 1, 1, 16) F(8, 1, 2, 16) F(8, 2, 3, 8) F(16, 1, 1, 8) F(16, 1, 2, 8)
+    F(2, 1, 1, 16) F(2, 1, 2, 16) F(2, 2, 2, 16) F(2, 2, 4, 16) F(2, 4, 6, 8) F(2, 4, 8, 8) \
+    F(4, 1, 1, 16) F(4, 1, 2, 16) F(4, 2, 2, 16) F(4, 3, 3, 8) F(4, 2, 6, 8) F(4, 4, 4, 8) \
+    F(8, 1, 1, 16) F(8, 1, 2, 16) F(8, 2, 3, 8) F(8, 2, 4, 8) F(16, 1, 1, 8) F(16, 1, 2, 8)
 
 // The field kind takes three words per voxel.
 #define TF_RESIDENT_SHAPES_FIELD(F) \
@@ -721,8 +755,10 @@ static int dispatch_resident(const tf_resident& p, const ResidentArgs& a, hipStr
         TF_RESIDENT_SHAPES_FIELD(F)
     } else if constexpr (KIND == TF_KIND_MULTIPHASE_FACES) {
         TF_RESIDENT_SHAPES_FACES(F)
-    } else {
+    } else if constexpr (KIND == TF_KIND_SOLVER) {
         TF_RESIDENT_SHAPES(F)
+    } else {
+        TF_RESIDENT_SHAPES_PAIRS(F)
     }
 #undef F
     return fail(-1, "resident shape (%d, %d, %d, %d) is not compiled", p.elems, p.px, p.py, p.waves);

@@ -41,8 +41,8 @@ def test_solver_shapes(shape):
     ((100, 60, 9), (2, 1, 2, 16)), ((120, 72, 9), (2, 2, 2, 16)), ((130, 130, 9), (2, 2, 4, 16)),
     ((230, 138, 9), (2, 4, 4, 16)), ((330, 198, 9), (2, 6, 8, 8)), ((100, 60, 140), (4, 1, 2, 16)),
     ((120, 72, 140), (4, 2, 2, 16)), ((130, 130, 140), (4, 2, 3, 16)), ((215, 129, 140), (4, 2, 4, 16)),
-    ((230, 138, 140), (4, 4, 5, 8)), ((270, 162, 140), (4, 4, 6, 8)), ((100, 60, 260), (8, 1, 2, 16)),
-    ((150, 90, 260), (8, 2, 2, 16)), ((120, 72, 260), (8, 2, 3, 8)), ((130, 130, 260), (8, 3, 4, 8)),
+    ((230, 138, 140), (4, 4, 6, 8)), ((290, 174, 140), (4, 4, 8, 8)), ((420, 252, 5), (2, 8, 8, 8)),
+    ((100, 60, 260), (8, 1, 2, 16)), ((150, 90, 260), (8, 2, 2, 16)), ((120, 72, 260), (8, 2, 3, 8)), ((130, 130, 260), (8, 3, 4, 8)),
     ((100, 60, 520), (16, 2, 2, 8))])
 def test_every_patch(shape, plan):
     img = _binary(shape, 5)
@@ -59,6 +59,17 @@ def test_images(shape):
     s = tau.Solver(img)
     assert s._resident_sweep() and s._resident.plan.lane_y
     _same(s, OracleSolver(img), 109 if shape[0] > 1 else 57)
+
+
+@pytest.mark.parametrize("shape", [(20, 21, 22), (120, 72, 9), (130, 130, 9)])
+def test_resumed_on_the_other_colour(shape):
+    """A launch that starts on an odd iteration (patches with even sides have
+    a kernel per first colour)."""
+    img = _binary(shape, 8)
+    s, o = tau.Solver(img), OracleSolver(img)
+    _same(s, o, 5)
+    s.solve(iter_limit=9, verbose=False, conv_crit=0.0)
+    assert s._resident and np.array_equal(s.field.cpu().numpy(), o.run(4).field.numpy())
 
 
 def test_batch():
@@ -187,8 +198,9 @@ D7 = {0: 0.0, 1: 1.0, 2: 0.5, 3: 0.25, 4: 0.12, 5: 2.0, 6: 1 / 3}
     ((3, 4, 5), (2, 1, 1, 16)), ((9, 8, 127), (2, 1, 1, 16)), ((100, 60, 5), (2, 1, 2, 16)),
     ((120, 72, 5), (2, 2, 2, 16)), ((130, 130, 5), (2, 2, 4, 16)), ((230, 138, 5), (2, 4, 6, 8)),
     ((7, 5, 140), (4, 1, 1, 16)), ((100, 60, 140), (4, 1, 2, 16)), ((120, 72, 140), (4, 2, 2, 16)),
-    ((130, 130, 140), (4, 3, 3, 8)), ((185, 111, 140), (4, 3, 4, 8)), ((6, 3, 260), (8, 1, 1, 16)),
-    ((100, 60, 260), (8, 1, 2, 16)), ((120, 72, 260), (8, 2, 3, 8)), ((6, 3, 520), (16, 1, 1, 8)),
+    ((130, 130, 140), (4, 3, 3, 8)), ((185, 111, 140), (4, 2, 6, 8)), ((215, 129, 140), (4, 4, 4, 8)),
+    ((290, 174, 5), (2, 4, 8, 8)), ((6, 3, 260), (8, 1, 1, 16)), ((100, 60, 260), (8, 1, 2, 16)),
+    ((120, 72, 260), (8, 2, 3, 8)), ((150, 90, 260), (8, 2, 4, 8)), ((6, 3, 520), (16, 1, 1, 8)),
     ((60, 36, 520), (16, 1, 2, 8))])
 def test_multiphase_every_patch(shape, plan):
     img = _labels(shape, 3, 7)
