@@ -37,7 +37,7 @@
 extern "C" {
 #endif
 
-#define TF_ABI_VERSION 16
+#define TF_ABI_VERSION 17
 
 #define TF_KIND_SOLVER 0
 #define TF_KIND_MULTIPHASE 1
@@ -71,6 +71,11 @@ extern "C" {
  * floats.  Prefactors must lie in [2^-20, 2^20].  Same iterates as
  * TF_KIND_MULTIPHASE. */
 #define TF_KIND_MULTIPHASE_FACES 5
+/* TF_KIND_SOLVER with its codes in groups of four rows (tf_pack_sweep_groups):
+ * one load brings the codes of several rows.  tf_sweep only, closed y and z,
+ * n_half 4 or 6, workgroups of 16 x 2 or 12 x 4 (waves x rows).  Same
+ * iterates as TF_KIND_SOLVER. */
+#define TF_KIND_SOLVER_GROUPS 6
 #define TF_MPF_MAX_CLASSES 4
 #define TF_MPF_FACE_SLOTS 16
 #define TF_MPF_MAX_FACTORS 2047
@@ -211,6 +216,17 @@ long long tf_sweep_codes_bytes(int X, int Y, int Z);
  * the other kinds the code itself.  */
 int tf_pack_sweep_codes(const uint8_t* codes, uint8_t* sweep_codes, int kind, int B, int X, int Y,
                         int Z, void* stream);
+
+/* The Solver codes in groups of four rows, for TF_KIND_SOLVER_GROUPS: 8 bytes
+ * hold the padded rows y = 4q-1 .. 4q+2 and the voxels z = 2p+1, 2p+2, byte
+ * 2r + e the count times 8 of row r and voxel e (0 past the padded volume);
+ * p in [0, (Z+1)/2) runs fastest, then q in [0, (Y+2)/4], then x in [0, X+1].
+ * No reference counterpart. */
+long long tf_sweep_groups_bytes(int X, int Y, int Z);
+
+/* Repack codes (set up for TF_KIND_SOLVER) into that layout, B consecutive
+ * volumes of tf_sweep_groups_bytes each; groups is 8-byte aligned. */
+int tf_pack_sweep_groups(const uint8_t* codes, uint8_t* groups, int B, int X, int Y, int Z, void* stream);
 
 /* Face codes of a labelled volume for tf_sweep with TF_KIND_MULTIPHASE_FACES
  * (layout at TF_KIND_MULTIPHASE_FACES).  No reference counterpart as an

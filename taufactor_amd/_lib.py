@@ -11,7 +11,7 @@ import threading
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libtauhip.so")
-ABI_VERSION = 16
+ABI_VERSION = 17
 
 KIND_SOLVER = 0
 KIND_MULTIPHASE = 1
@@ -20,6 +20,8 @@ KIND_ANISOTROPIC = 3
 ANISO_TABLE = 147
 KIND_ELECTRODE = 4
 KIND_MULTIPHASE_FACES = 5
+KIND_SOLVER_GROUPS = 6
+GROUP_DEPTHS = (4, 6)  # its compiled half-sweeps per pass
 MPF_MAX_CLASSES = 4
 MPF_FACE_SLOTS = 16
 MPF_MAX_FACTORS = 2047
@@ -67,6 +69,8 @@ SIGNATURES = {
     "tf_wrap_ghosts": (_c_int, [_vp, _c_int, _c_int, _c_int, _c_int, _vp]),
     "tf_wrap_ghosts_from": (_c_int, [_vp, _vp, _c_int, _c_int, _c_int, _c_int, _vp]),
     "tf_sweep_codes_bytes": (ctypes.c_longlong, [_c_int, _c_int, _c_int]),
+    "tf_sweep_groups_bytes": (ctypes.c_longlong, [_c_int, _c_int, _c_int]),
+    "tf_pack_sweep_groups": (_c_int, [_vp, _vp, _c_int, _c_int, _c_int, _c_int, _vp]),
     "tf_pack_sweep_codes": (_c_int, [_vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_int, _vp]),
     "tf_multiphase_face_codes": (_c_int, [_vp, _vp, _c_int, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _vp]),
     "tf_sweep": (_c_int, [_vp, _vp, _vp, _vp, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,

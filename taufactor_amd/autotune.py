@@ -34,6 +34,8 @@ TIMED_LAUNCHES = 6
 SOLVER_SPACE = ((5, 4, 6, 3, 2), ((16, 2), (12, 2), (8, 2)), (0, 128, 64))
 FIELD_SPACE = ((4, 3, 2), ((8, 2), (12, 2), (16, 2)), (0, 128, 64))
 BATCH_SPACE = ((5, 4, 6, 2), ((8, 2), (4, 4), (12, 2), (16, 2)), (64, 32))
+# closed Solver volumes keep their codes in groups of four rows for these as well
+GROUP_SPACE = ((6, 4), ((12, 4),), (0,))
 TIE = 0.02
 
 _cache: dict = {}
@@ -89,7 +91,7 @@ def tune_solver(s, fixed_h=None, fixed_tile=None):
     B, X, Y, Z = s.batch_size, s.Nx, s.Ny, s.Nz
     # the kind, codes and table the solver's own launches use (MultiPhase
     # volumes may sweep through face codes instead of class codes)
-    kind, codes, hm, n_table = s._sweep_pointers()
+    kind, _, _, n_table = s._sweep_pointers()
     key = ("plain", kind, n_table, B, X, Y, Z, fixed_h, None if fixed_tile is None else tuple(fixed_tile))
     if key in _cache:
         return _cache[key]
@@ -102,8 +104,11 @@ def tune_solver(s, fixed_h=None, fixed_tile=None):
     dst.copy_(s.field)
     stream = s._stream()
     timings = []
-    for H, tile in _candidates(space, fixed_h, fixed_tile):
-        t = _lib.Tile(*tile)
+    candidates = _candidates(space, fixed_h, fixed_tile)
+    if fixed_tile is None and s._sweep_groups() is not None:
+        candidates += [c for c in _candidates(GROUP_SPACE, fixed_h, None) if c[0] in _lib.GROUP_DEPTHS]
+    for H, tile in candidates:
+        kind, codes, hm, n_table, t = s._launch_operands(H, _lib.Tile(*tile))
         bufs = [src, dst]
         state = {"i": 0}
 

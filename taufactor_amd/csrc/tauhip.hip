@@ -411,6 +411,51 @@ extern "C" int tf_pack_sweep_codes(const uint8_t* codes, uint8_t* sweep_codes, i
     return 0;
 }
 
+// One group of sweep_group_volume per lane: a read of the codes' bytes and one
+// 8-byte store (512^3: 127 us at 2.1 TB/s; run once per
+// volume)
+__global__ void k_pack_sweep_groups(const uint8_t* __restrict__ codes, uint2* __restrict__ out, Vol v,
+                                    long long n) {
+    const long long gid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (gid >= n) return;
+    const int nP = group_pairs(v.Z), nQ = group_rows(v.Y);
+    const int p = (int)(gid % nP);
+    const long long row = gid / nP;
+    const int q = (int)(row % nQ);
+    const uint8_t* src = codes + (row / nQ) * (long long)v.sX;
+    uint32_t w[2] = {0, 0};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int y = 4 * q - 1 + r;
+        if (y < 0 || y > v.Y + 1) continue;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const uint32_t c = src[y * v.sY + 2 * p + 1 + e];  // z <= Z + 1
+            w[r >> 1] |= (c << 3) << (16 * (r & 1) + 8 * e);
+        }
+    }
+    out[gid] = make_uint2(w[0], w[1]);
+}
+
+extern "C" long long tf_sweep_groups_bytes(int X, int Y, int Z) {
+    if (X < 1 || Y < 1 || Z < 1) return fail(-1, "invalid shape %dx%dx%d", X, Y, Z);
+    return sweep_group_volume(X, Y, Z);
+}
+
+extern "C" int tf_pack_sweep_groups(const uint8_t* codes, uint8_t* groups, int B, int X, int Y, int Z,
+                                    void* stream) {
+    if (int rc = check_dims(B, X, Y, Z)) return rc;
+    if (!codes || !groups) return fail(-1, "null pointer argument");
+    if (reinterpret_cast<uintptr_t>(groups) & 7) return fail(-1, "groups must be 8-byte aligned");
+    const long long n = (long long)B * sweep_group_volume(X, Y, Z) / 8;
+    const long long blocks = (n + 255) / 256;
+    if (blocks >= (1LL << 31)) return fail(-1, "volume too large");
+    hipLaunchKernelGGL(k_pack_sweep_groups, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, codes,
+                       reinterpret_cast<uint2*>(groups), make_vol(X, Y, Z), n);
+    TF_LAUNCH_CHECK("k_pack_sweep_groups");
+    return 0;
+}
+
 // ---------------------------------------------------------------------------
 // unblocked in-place half-sweep: one thread per interior voxel
 // ---------------------------------------------------------------------------
@@ -476,7 +521,8 @@ extern "C" int tf_sweep_half_inplace(float* field, const uint8_t* codes, const f
 // n_half <= 4) and the volume is tall enough; the x-tile length is left to
 // the launch (balanced_tx).  Any shape gives identical results.
 static void default_tile(int H, int kind, int Y, tf_tile* t) {
-    const bool tall = (own_code_kind(kind) || (kind != TF_KIND_FIELD && H <= 4)) && Y >= 64;
+    const bool tall = kind == TF_KIND_SOLVER_GROUPS ||
+                      ((own_code_kind(kind) || (kind != TF_KIND_FIELD && H <= 4)) && Y >= 64);
     t->waves = tall ? 16 : 8;
     t->rows_per_wave = 2;
     t->tx = 0;  // chosen at launch from the resident workgroups (balanced_tx)
@@ -503,7 +549,8 @@ static int sweep_prepare(const float* hm_lut, int n_classes, int kind, int B, in
                          int n_half, const tf_tile* tile, tf_tile* t) {
     if (int rc = check_dims(B, X, Y, Z)) return rc;
     if (kind != TF_KIND_SOLVER && kind != TF_KIND_MULTIPHASE && kind != TF_KIND_FIELD &&
-        kind != TF_KIND_ANISOTROPIC && kind != TF_KIND_ELECTRODE && kind != TF_KIND_MULTIPHASE_FACES)
+        kind != TF_KIND_ANISOTROPIC && kind != TF_KIND_ELECTRODE && kind != TF_KIND_MULTIPHASE_FACES &&
+        kind != TF_KIND_SOLVER_GROUPS)
         return fail(-1, "unknown kind %d", kind);
     if (kind == TF_KIND_MULTIPHASE_FACES &&
         (!hm_lut || n_classes < TF_MPF_FACE_SLOTS + 2 || n_classes > TF_MPF_FACE_SLOTS + 2 * TF_MPF_MAX_FACTORS + 2))
@@ -536,6 +583,8 @@ static int sweep_dispatch(int kind, int n_half, SweepArgs& a, int B, const tf_ti
                           hipStream_t st) {
     if (kind == TF_KIND_SOLVER)
         return sweep_dispatch_solver(n_half, a, B, t.waves, t.rows_per_wave, st);
+    if (kind == TF_KIND_SOLVER_GROUPS)
+        return sweep_dispatch_solver_groups(n_half, a, B, t.waves, t.rows_per_wave, st);
     if (kind == TF_KIND_MULTIPHASE)
         return sweep_dispatch_multiphase(n_half, a, B, t.waves, t.rows_per_wave, st);
     if (kind == TF_KIND_MULTIPHASE_FACES)

@@ -31,8 +31,9 @@
 // counts half-sweeps across launches, written and read with relaxed
 // device-scope atomics, so no flag, fence or second round trip follows the
 // data: 1.0 to 1.3 us from the update of a border row to its use in another
-// workgroup.  Two slots per row suffice: a wave sends half-sweep t + 1's rows after it has read its partner's of t,
-// which the partner sent after reading the slot that is written again.
+// workgroup.  Two slots per row suffice: a wave sends half-sweep t + 1's rows after
+// it has read its partner's of t, which the partner sent after reading the
+// slot that is written again.
 //
 // Progress.  The workgroups wait for each other, so all of them have to be
 // resident: the launch checks the grid against the occupancy.  Other work on
@@ -68,6 +69,19 @@ struct ResidentArgs {
 };
 
 constexpr int kResidentSpin = 1 << 16;  // polls of one wait, about 50 ms
+
+// (1/f, f) of a prefactor table entry for the reciprocal division of the
+// anisotropic and electrode kinds; inf (an inert voxel) is the pair (0, 0).
+// q = s (1/f) and one residual correction is s / f correctly rounded for a
+// correctly rounded 1/f, f in [2^-20, 2^20] and |s| >= 2^-100 (Markstein's
+// correction step: the residual is exact); `odd` reports a prefactor outside
+// that range (a NaN among them), for which a launch divides throughout.
+__device__ __forceinline__ void prefactor_pair(float f, float& r, float& g, bool& odd) {
+    const bool inert = f == __builtin_inff();
+    odd = !inert && !(f >= 0x1p-20f && f <= 0x1p20f);
+    r = inert ? 0.0f : 1.0f / f;
+    g = inert ? 0.0f : f;
+}
 
 template <int KIND>
 constexpr int resident_table_floats() {

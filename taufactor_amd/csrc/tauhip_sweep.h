@@ -66,6 +66,15 @@ __host__ __device__ inline long long sweep_code_volume(int X, int Y, int Z) {
     return (long long)(X + 2) * (Y + 2) * sweep_code_row(Z);
 }
 
+// sweep codes in groups of four rows (TF_KIND_SOLVER_GROUPS): 8 bytes hold
+// rows 4q-1 .. 4q+2 (padded y) x z = 2p+1, 2p+2, byte 2r + e the code of row
+// r, element e; p fastest, then q, then x in [0, X+1]
+__host__ __device__ inline int group_rows(int Y) { return (Y + 2) / 4 + 1; }
+__host__ __device__ inline int group_pairs(int Z) { return (Z + 1) / 2; }
+__host__ __device__ inline long long sweep_group_volume(int X, int Y, int Z) {
+    return 8LL * (X + 2) * group_rows(Y) * group_pairs(Z);
+}
+
 static inline int check_dims(int B, int X, int Y, int Z) {
     if (B < 1 || X < 1 || Y < 1 || Z < 1)
         return fail(-1, "invalid volume shape B=%d X=%d Y=%d Z=%d", B, X, Y, Z);
@@ -116,19 +125,6 @@ __device__ __forceinline__ float div_by_count(float s, float r, float d, int cod
     q = __builtin_fmaf(e, r, q);
     if (__builtin_amdgcn_classf(e, 0x90)) q = s / d;
     return q;
-}
-
-// (1/f, f) of a prefactor table entry for the reciprocal division of the
-// anisotropic and electrode kinds; inf (an inert voxel) is the pair (0, 0).
-// q = s (1/f) and one residual correction is s / f correctly rounded for a
-// correctly rounded 1/f, f in [2^-20, 2^20] and |s| >= 2^-100 (Markstein's
-// correction step: the residual is exact); `odd` reports a prefactor outside
-// that range (a NaN among them), for which a launch divides throughout.
-__device__ __forceinline__ void prefactor_pair(float f, float& r, float& g, bool& odd) {
-    const bool inert = f == __builtin_inff();
-    odd = !inert && !(f >= 0x1p-20f && f <= 0x1p20f);
-    r = inert ? 0.0f : 1.0f / f;
-    g = inert ? 0.0f : f;
 }
 
 // table of (1/d, d) per Solver code; code 0 means factor = inf
@@ -389,7 +385,7 @@ __device__ __forceinline__ float from_next_lane(uint32_t v) {
 // not).  The other kinds allocate nothing here.
 template <int KIND>
 __device__ __forceinline__ float* code_table() {
-    if constexpr (KIND == TF_KIND_SOLVER) {
+    if constexpr (KIND == TF_KIND_SOLVER || KIND == TF_KIND_SOLVER_GROUPS) {
         __shared__ __align__(16) float t[18];
         return t;
     } else if constexpr (KIND == TF_KIND_ANISOTROPIC) {
@@ -430,6 +426,17 @@ __device__ __forceinline__ void rsweep_tile(const float* __restrict__ S, float* 
     // layout (byte offsets of the x+, y+, z+ face conductances and of the
     // (1/f, f) prefactor pair), hm the face table and the pairs
     constexpr bool kFaceCodes = KIND == TF_KIND_MULTIPHASE_FACES;
+    // Solver codes in groups of four rows: one load brings the codes of four
+    // rows' pairs (two rows' where the wave's rows straddle two groups), and
+    // the ring holds two rows in a register.  A vector memory instruction
+    // costs about as much as the bytes it moves: one 2-byte load per row and
+    // plane was a sixth of the 512^3 launch (16 x 2, H = 6: 58.0 -> 54.0 us per
+    // half-sweep), and the registers saved let a wave hold four rows
+    constexpr bool kGroups = KIND == TF_KIND_SOLVER_GROUPS;
+    static_assert(!kGroups || H % 2 == 0, "a row pair starts at an odd y");
+    // the wave's four rows are one group
+    constexpr bool kQuad = kGroups && RPW == 4 && (2 - H) % 4 == 0 && Sh::TY % 4 == 0;
+    constexpr int NQ = kGroups ? Sh::NR : 1;
     constexpr int NG = kFaces ? Sh::NR : 1;
     constexpr int NKF = kFaceCodes ? Sh::NR : 1;
     constexpr int TY = Sh::TY, ML = Sh::ML, NR = Sh::NR, DP = Sh::D, EB = Sh::EB;
@@ -456,7 +463,7 @@ __device__ __forceinline__ void rsweep_tile(const float* __restrict__ S, float* 
     const int lx1 = min(x1 + H, v.X + 2);
 
     float* const s_code = code_table<KIND>();
-    if (KIND == TF_KIND_SOLVER) {
+    if (KIND == TF_KIND_SOLVER || KIND == TF_KIND_SOLVER_GROUPS) {
         if (threadIdx.x < 18) s_code[threadIdx.x] = c_rd[threadIdx.x];
     } else if (KIND == TF_KIND_ANISOTROPIC) {
         if (threadIdx.x < TF_ANISO_TABLE) s_code[threadIdx.x] = hm[threadIdx.x];
@@ -493,8 +500,8 @@ __device__ __forceinline__ void rsweep_tile(const float* __restrict__ S, float* 
     const uint32_t span_f = (uint32_t)(lx1 - pbase) * (uint32_t)plane_f;
     const rsrc_t rF = make_rsrc(reinterpret_cast<const char*>(S + (size_t)pbase * v.sX) - kSlackBytes,
                                 span_f + 2u * kSlackBytes);
-    const int row_c = sweep_code_row(v.Z);
-    const int plane_c = (v.Y + 2) * row_c;
+    const int row_c = kGroups ? 8 * group_pairs(v.Z) : sweep_code_row(v.Z);
+    const int plane_c = (kGroups ? group_rows(v.Y) : v.Y + 2) * row_c;
     const rsrc_t rC = make_rsrc(Cg + (size_t)pbase * plane_c, (uint32_t)(lx1 - pbase) * (uint32_t)plane_c);
     // face codes: one descriptor over the uint32 array, laid out (and
     // offset) like the field
@@ -537,8 +544,16 @@ __device__ __forceinline__ void rsweep_tile(const float* __restrict__ S, float* 
             ys[k][j] = own_row[k][j] ? yk : 0;
         }
     }
+    int vq[RPW / 2];  // code groups: offset of each row pair's codes
+#pragma unroll
+    for (int j = 0; j < RPW / 2; ++j) {
+        const int r = ey0 + wave * RPW + 2 * j + 1;  // even: the first row's place in the groups
+        const bool ok = kGroups && r >= 0 && (r >> 2) < group_rows(v.Y) && zl >= 1 && zl <= v.Z;
+        vq[j] = ok ? (r >> 2) * row_c + (zl >> 1) * 8 + (r & 2) * 2 : kOff;
+    }
     u32x2_t F[NR][RPW];
     uint32_t K[NR][RPW];
+    uint32_t KP[NQ][RPW / 2];
     u32x2_t G[NG][RPW][3];  // field kind: gx, gy, gz pairs
     u32x2_t KF[NKF][RPW];   // face codes of the lane's pair
     // slots the prologue does not load hold planes before the stream start
@@ -550,6 +565,10 @@ __device__ __forceinline__ void rsweep_tile(const float* __restrict__ S, float* 
             F[i][j] = u32x2_t{0u, 0u};
             K[i][j] = 0u;
         }
+#pragma unroll
+    for (int i = 0; i < NQ; ++i)
+#pragma unroll
+        for (int j = 0; j < RPW / 2; ++j) KP[i][j] = 0u;
 #pragma unroll
     for (int i = 0; i < NG; ++i)
 #pragma unroll
@@ -567,10 +586,18 @@ __device__ __forceinline__ void rsweep_tile(const float* __restrict__ S, float* 
     // record counts below 2^31 (a tile's planes span less than 2 GiB)
     const int rec_f = (int)(span_f + 2u * kSlackBytes);
     const int rec_c = (int)((uint32_t)(lx1 - pbase) * (uint32_t)plane_c);
-    auto issue_load = [&](int p, auto slot_c) {
+    auto issue_load = [&](int p, auto slot_c) __attribute__((always_inline)) {
         constexpr int sl = decltype(slot_c)::value;
         const bool pok = p >= pbase && p < lx1;
         const int sf = pok ? (p - pbase) * plane_f : rec_f, sc = pok ? (p - pbase) * plane_c : rec_c;
+        if constexpr (kQuad) {
+            const u32x2_t k = __builtin_amdgcn_raw_buffer_load_b64(rC, vq[0], sc, 0);
+            KP[sl][0] = k.x;
+            KP[sl][1] = k.y;
+        } else if constexpr (kGroups) {
+#pragma unroll
+            for (int j = 0; j < RPW / 2; ++j) KP[sl][j] = __builtin_amdgcn_raw_buffer_load_b32(rC, vq[j], sc, 0);
+        }
 #pragma unroll
         for (int j = 0; j < RPW; ++j) {
             F[sl][j] = __builtin_amdgcn_raw_buffer_load_b64(rF, vf[j], sf, 0);
@@ -580,7 +607,7 @@ __device__ __forceinline__ void rsweep_tile(const float* __restrict__ S, float* 
                     G[sl][j][k] = __builtin_amdgcn_raw_buffer_load_b64(rG[k], vf[j], sf, 0);
             } else if constexpr (kFaceCodes) {
                 KF[sl][j] = __builtin_amdgcn_raw_buffer_load_b64(rK, vf[j], sf, 0);
-            } else {
+            } else if constexpr (!kGroups) {
                 K[sl][j] = __builtin_amdgcn_raw_buffer_load_b16(rC, vc[j], sc, 0);
             }
         }
@@ -604,7 +631,7 @@ __device__ __forceinline__ void rsweep_tile(const float* __restrict__ S, float* 
         const bool own = (half ? own_row[1][j] : own_row[0][j]) && zl >= z0 && zl < z1;
         so[j] = own ? ((half ? ys[1][j] : ys[0][j]) * v.sY + zl) * 4 : kOff;
     }
-    auto store_plane = [&](int q, auto slot_c) {
+    auto store_plane = [&](int q, auto slot_c) __attribute__((always_inline)) {
         constexpr int sl = decltype(slot_c)::value;
         const bool qok = q >= x0 && q < x1;
         const rsrc_t r = make_rsrc(D + (size_t)(qok ? q : 0) * v.sX, qok ? (uint32_t)(4 * v.sX) : 0u);
@@ -645,13 +672,13 @@ __device__ __forceinline__ void rsweep_tile(const float* __restrict__ S, float* 
     // parity of step s is that of S0 + u, S0 having the parity of H
     auto ebuf = [&](int h, int par) { return eb + (h * 2 + par) * EB; };
 
-    auto body = [&](auto a_c) {
+    auto body = [&](auto a_c) __attribute__((always_inline)) {
         constexpr int AA = decltype(a_c)::value;
         // active element (0: z = zl, 1: z = zl + 1) of row j at step u
         auto act = [](int u, int j) { return (AA ^ (u + j)) & 1; };
         auto par = [](int u) { return (H + u) & 1; };
 
-        auto publish = [&](int h, int u, auto slot_c) {
+        auto publish = [&](int h, int u, auto slot_c) __attribute__((always_inline)) {
             constexpr int sl = decltype(slot_c)::value;
             float* e = ebuf(h, par(u));
             const int a0 = act(u, 0), a1 = act(u, RPW - 1);
@@ -661,7 +688,7 @@ __device__ __forceinline__ void rsweep_tile(const float* __restrict__ S, float* 
         // field kind: the y faces of the last row of a freshly loaded plane,
         // read by the first row of the wave below in every half-sweep of
         // that plane (LDS ring slot = register ring slot)
-        auto publish_faces = [&](auto slot_c) {
+        auto publish_faces = [&](auto slot_c) __attribute__((always_inline)) {
             constexpr int sl = decltype(slot_c)::value;
             if constexpr (kFaces) {
                 reinterpret_cast<u32x2_t*>(sGE + sl * Sh::GEB)[(wave + 1) * kRowPairs + lane] =
@@ -684,7 +711,7 @@ __device__ __forceinline__ void rsweep_tile(const float* __restrict__ S, float* 
 
         // chk: test the plane bounds of the half-sweep (the steady-state
         // blocks, where every plane of every half-sweep is in bounds, skip it)
-        auto stage = [&](auto h_c, auto u_c, int p, auto chk_c) {
+        auto stage = [&](auto h_c, auto u_c, int p, auto chk_c) __attribute__((always_inline)) {
             constexpr int h = decltype(h_c)::value, u = decltype(u_c)::value;
             constexpr int sl = ((u - h + 1) % NR + NR) % NR;
             constexpr int slm = (sl + NR - 1) % NR, slp = (sl + 1) % NR;
@@ -706,6 +733,18 @@ __device__ __forceinline__ void rsweep_tile(const float* __restrict__ S, float* 
                 // face codes: the y+ face offsets of the last row above
                 ka = sKE[sl * Sh::KEB + lane + wave * 2 * kRowPairs + kRowPairs];
             }
+            // code groups: the codes are unpacked anew in each half-sweep (else
+            // the compiler keeps every unpacked code of the ring in a
+            // register), and one test for rare quotients serves all rows
+            float q[RPW], sum[RPW];
+            bool any_rare = false;
+            auto code_of = [&](int j) {
+                return (KP[kGroups ? sl : 0][j / 2] >> (16 * (j & 1) + 8 * act(u, j))) & 0xffu;
+            };
+            if constexpr (kGroups) {
+#pragma unroll
+                for (int j = 0; j < RPW / 2; ++j) asm("" : "+v"(KP[sl][j]));
+            }
 #pragma unroll
             for (int j = 0; j < RPW; ++j) {
                 const int a = act(u, j);
@@ -720,7 +759,21 @@ __device__ __forceinline__ void rsweep_tile(const float* __restrict__ S, float* 
                 // Solver: the byte is 8 x the count, the offset of its table entry
                 const uint32_t code = a ? (K[sl][j] >> 8) : (K[sl][j] & 0xffu);
                 float out;
-                if constexpr (KIND == TF_KIND_SOLVER) {
+                if constexpr (kGroups) {
+                    const float2 rdv =
+                        *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(s_code) + code_of(j));
+                    float s = xp + xm;
+                    s = s + yp;
+                    s = s + ym;
+                    s = s + zp;
+                    s = s + zm;
+                    const float qt = s * rdv.x;
+                    const float e2 = __builtin_fmaf(-qt, rdv.y, s);
+                    q[j] = __builtin_fmaf(e2, rdv.x, qt);
+                    sum[j] = s;
+                    any_rare = any_rare || __builtin_amdgcn_classf(e2, 0x90);
+                    continue;
+                } else if constexpr (KIND == TF_KIND_SOLVER) {
                     const float2 rdv =
                         *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(s_code) + code);
                     float s = xp + xm;
@@ -846,11 +899,33 @@ __device__ __forceinline__ void rsweep_tile(const float* __restrict__ S, float* 
                 else
                     F[sl][j].x = __builtin_bit_cast(uint32_t, out);
             }
+            if constexpr (kGroups) {
+                // (the IEEE division gives the other rows the quotient they have)
+                if (__builtin_expect(__builtin_amdgcn_ballot_w64(any_rare) != 0, 0)) {
+#pragma unroll
+                    for (int j = 0; j < RPW; ++j) {
+                        const uint32_t code = code_of(j);
+                        q[j] = sum[j] / (code ? (float)(code >> 3) : __builtin_inff());
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < RPW; ++j) {
+                    const int a = act(u, j);
+                    const float c = a ? hi_f(F[sl][j]) : lo_f(F[sl][j]);
+                    float s = q[j] - c;
+                    s = s * w;
+                    const float out = c + s;
+                    if (a)
+                        F[sl][j].y = __builtin_bit_cast(uint32_t, out);
+                    else
+                        F[sl][j].x = __builtin_bit_cast(uint32_t, out);
+                }
+            }
         };
 
         // planes S0-1 .. S0+1+DP in flight; plane S0's edges published as
         // "step S0-1" for the first half-sweep
-        static_for<0, DP + 3>([&](auto i_c) {
+        static_for<0, DP + 3>([&](auto i_c) __attribute__((always_inline)) {
             constexpr int i = decltype(i_c)::value;
             issue_load(S0 - 1 + i, ic<i>{});
         });
@@ -859,11 +934,11 @@ __device__ __forceinline__ void rsweep_tile(const float* __restrict__ S, float* 
         __syncthreads();
 
         // one block of NR steps from s0 (ring slots are compile-time in u)
-        auto block = [&](int s0, auto chk_c) {
-            static_for<0, NR>([&](auto u_c) {
+        auto block = [&](int s0, auto chk_c) __attribute__((always_inline)) {
+            static_for<0, NR>([&](auto u_c) __attribute__((always_inline)) {
                 constexpr int u = decltype(u_c)::value;
                 const int s = s0 + u;
-                static_for<0, H>([&](auto h_c) {
+                static_for<0, H>([&](auto h_c) __attribute__((always_inline)) {
                     constexpr int h = decltype(h_c)::value;
                     stage(h_c, u_c, s - h, chk_c);
                     if constexpr (h + 1 < H) publish(h + 1, u, ic<((u - h + 1) % NR + NR) % NR>{});
@@ -888,7 +963,7 @@ __device__ __forceinline__ void rsweep_tile(const float* __restrict__ S, float* 
         }
         if (skips) s_hi = s_lo - 1;
         int s0 = S0;
-        if constexpr (KIND == TF_KIND_SOLVER) {
+        if constexpr (KIND == TF_KIND_SOLVER || KIND == TF_KIND_SOLVER_GROUPS) {
             // the Solver kind (plain and batched) runs the steady-state blocks
             // without the bounds tests (512^3: 0.402 -> 0.385 ms per launch);
             // the kinds with more live registers per update spill in that
@@ -928,7 +1003,9 @@ __global__ __launch_bounds__(NW * 64) void k_sweep(SweepArgs a) {
     const uint8_t* codes =
         KIND == TF_KIND_FIELD || KIND == TF_KIND_MULTIPHASE_FACES
             ? reinterpret_cast<const uint8_t*>(static_cast<const float*>(a.codes) + off)
-            : static_cast<const uint8_t*>(a.codes) + (size_t)b * sweep_code_volume(a.v.X, a.v.Y, a.v.Z);
+            : static_cast<const uint8_t*>(a.codes) +
+                  (size_t)b * (KIND == TF_KIND_SOLVER_GROUPS ? sweep_group_volume(a.v.X, a.v.Y, a.v.Z)
+                                                             : sweep_code_volume(a.v.X, a.v.Y, a.v.Z));
     const float* hm = KIND == TF_KIND_ELECTRODE ? a.hm + (size_t)b * TF_ELECTRODE_TABLE : a.hm;
     rsweep_tile<H, KIND, NW, RPW, AA>(a.src + off, a.dst + off, codes, hm, a.v, a.w, a.TX,
                                   nar ? a.z0N : 1 + tz * RegShape<H, NW, RPW>::TZ, ty, tx, nar,
@@ -952,7 +1029,7 @@ static size_t sweep_lds_bytes(int kind, int ncls) {
 // LDS of the kind's static table (code_table), with room for its alignment;
 // a launch needs it on top of the dynamic bytes
 static constexpr size_t static_table_bytes(int kind) {
-    return 64 + sizeof(float) * (kind == TF_KIND_SOLVER ? 18
+    return 64 + sizeof(float) * (kind == TF_KIND_SOLVER || kind == TF_KIND_SOLVER_GROUPS ? 18
                                  : kind == TF_KIND_ANISOTROPIC ? TF_ANISO_TABLE
                                  : kind == TF_KIND_ELECTRODE ? TF_ELECTRODE_TABLE
                                  : kind == TF_KIND_MULTIPHASE_FACES ? TF_MPF_FACE_SLOTS + 2 * TF_MPF_MAX_FACTORS + 2
@@ -1110,6 +1187,18 @@ static int dispatch_sweep(int H, SweepArgs& a, int B, int nw, int rpw, hipStream
     }
 }
 
+// Solver codes in groups: the depths and shapes that large volumes run
+template <int KIND>
+static int dispatch_groups(int H, SweepArgs& a, int B, int nw, int rpw, hipStream_t st) {
+    static_assert(KIND == TF_KIND_SOLVER_GROUPS, "");
+    if (H == 6 && nw == 16 && rpw == 2) return launch_sweep<6, KIND, 16, 2>(a, B, st);
+    if (H == 4 && nw == 16 && rpw == 2) return launch_sweep<4, KIND, 16, 2>(a, B, st);
+    if (H == 6 && nw == 12 && rpw == 4) return launch_sweep<6, KIND, 12, 4>(a, B, st);
+    if (H == 4 && nw == 12 && rpw == 4) return launch_sweep<4, KIND, 12, 4>(a, B, st);
+    return fail(-1, "workgroup shape %d waves x %d rows is not compiled for kind %d and n_half %d", nw, rpw, KIND,
+                H);
+}
+
 // ---------------------------------------------------------------------------
 // uneven batch: many two-phase volumes, each with its own convergence
 // ---------------------------------------------------------------------------
@@ -1265,6 +1354,7 @@ static int dispatch_batch_shape(BatchArgs& a, int nw, int rpw, hipStream_t st) {
 // ---------------------------------------------------------------------------
 // Launch (or, with a.resolve_only, only size) the sweep of one kind.
 int sweep_dispatch_solver(int H, SweepArgs& a, int B, int nw, int rpw, hipStream_t st);
+int sweep_dispatch_solver_groups(int H, SweepArgs& a, int B, int nw, int rpw, hipStream_t st);
 int sweep_dispatch_multiphase(int H, SweepArgs& a, int B, int nw, int rpw, hipStream_t st);
 int sweep_dispatch_mpfaces(int H, SweepArgs& a, int B, int nw, int rpw, hipStream_t st);
 int sweep_dispatch_field(int H, SweepArgs& a, int B, int nw, int rpw, hipStream_t st);

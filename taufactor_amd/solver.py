@@ -88,6 +88,7 @@ class SORSolver(ABC):
         self._launch_events = None  # list -> (start, end, n_launches) per _advance
         self._codes = None
         self._sweep_codes = None
+        self._groups = None  # see Solver._sweep_groups
         self._hm_lut = None
         self._n_classes = 0
         self._spans_cache = {}
@@ -271,6 +272,24 @@ class SORSolver(ABC):
             raise RuntimeError(f"the sweep table of kind {kind} needs {n_table} entries")
         return kind | self._sweep_flags, _lib.ptr(codes), _lib.ptr(table) if table is not None else None, n_table
 
+    def _sweep_groups(self):
+        """The sweep codes in groups of four rows, or None (see Solver)."""
+        return None
+
+    def _launch_operands(self, H: int, tile):
+        """(kind with the sweep flags, codes address, table address, table
+        length, tile) of a launch of H half-sweeps with `tile` (a _lib.Tile or
+        None): _sweep_pointers, or the codes in groups where a kernel for
+        them is compiled for this depth and workgroup shape."""
+        shape = (tile.waves, tile.rows_per_wave) if tile is not None else (16, 2) if self.Ny >= 64 else None
+        if H in _lib.GROUP_DEPTHS and (shape == (16, 2) or shape == (12, 4) and self.tile is None):
+            groups = self._sweep_groups()
+            if groups is not None:
+                return _lib.KIND_SOLVER_GROUPS, _lib.ptr(groups), None, 0, tile
+        if shape == (12, 4) and self.tile is None:
+            tile = None  # the last launch of a block: another depth
+        return (*self._sweep_pointers(), tile)
+
     def resolved_launch(self):
         """(H, (waves, rows_per_wave, tx), n_tiles) of the next sweep launches
         with every default resolved by the library (tf_sweep_launch_config)."""
@@ -278,7 +297,7 @@ class SORSolver(ABC):
         H = max(1, min(H, _lib.MAX_FUSED_HALF_SWEEPS))
         out, n = _lib.Tile(), ctypes.c_int(0)
         req = _lib.Tile(*tile) if tile is not None else None
-        kind, _, _, n_table = self._sweep_pointers()
+        kind, _, _, n_table, req = self._launch_operands(H, req)
         st = self._lib.tf_sweep_launch_config(kind, n_table, self.batch_size, self.Nx,
                                               self.Ny, self.Nz, H, req, ctypes.byref(out),
                                               ctypes.byref(n))
@@ -286,22 +305,21 @@ class SORSolver(ABC):
         return H, (out.waves, out.rows_per_wave, out.tx), n.value
 
     def _sweep_args(self):
-        """(per, tile, codes, hm) of the next sweep launches."""
+        """(per, tile) of the next sweep launches."""
         per, tile = self._launch_config()
         per = max(1, min(per, _lib.MAX_FUSED_HALF_SWEEPS))
         if tile is not None:
             tile = _lib.Tile(*tile)
-        # the sweep reads the aligned sweep codes (the face conductances for
-        # the field kind, the face codes for MultiPhase volumes that fit them)
-        _, codes, hm, _ = self._sweep_pointers()
-        return per, tile, codes, hm
+        return per, tile
 
-    def _launch(self, h: int, it: int, tile, codes, hm) -> None:
+    def _launch(self, h: int, it: int, tile) -> None:
         """One tf_sweep launch of h half-sweeps from iteration it (its colour)."""
         B, X, Y, Z = self.batch_size, self.Nx, self.Ny, self.Nz
         src = self._fields[self._cur]
         dst = self._fields[1 - self._cur]
-        kind, _, _, n_table = self._sweep_pointers()
+        # the sweep reads the aligned sweep codes (the face conductances for
+        # the field kind, the face codes for MultiPhase volumes that fit them)
+        kind, codes, hm, n_table, tile = self._launch_operands(h, tile)
         st = self._lib.tf_sweep(_lib.ptr(src), _lib.ptr(dst), codes, hm, n_table,
                                 kind, B, X, Y, Z, self._w32, it & 1, h,
                                 tile, self._stream())
@@ -317,7 +335,7 @@ class SORSolver(ABC):
         n_half -= done
         if n_half > 0 and resident and self._resident_sweep() and self._resident.launch(self, n_half, it):
             return
-        per, tile, codes, hm = self._sweep_args()
+        per, tile = self._sweep_args()
         # timing (bench.py): HIP events on the launch stream around the
         # launches that fuse the full `per` half-sweeps (a shorter last
         # launch is another kernel and is left out)
@@ -330,7 +348,7 @@ class SORSolver(ABC):
         launches = 0
         while n_half > 0:
             h = min(per, n_half)
-            self._launch(h, it, tile, codes, hm)
+            self._launch(h, it, tile)
             it += h
             n_half -= h
             launches += 1
@@ -364,7 +382,7 @@ class SORSolver(ABC):
             if self._resident.launch(self, n, self.iter):
                 self._ahead = n
                 return
-        per, tile, codes, hm = self._sweep_args()
+        per, tile = self._sweep_args()
         launches = 1
         if self._spare is not None:
             launches = self.MAX_AHEAD
@@ -377,7 +395,7 @@ class SORSolver(ABC):
             if i == 1:
                 k = 1 - self._cur  # the checked field, after the first launch
                 self._fields[k], self._spare = self._spare, self._fields[k]
-            self._launch(h, self.iter + done, tile, codes, hm)
+            self._launch(h, self.iter + done, tile)
             done += h
         self._ahead = done
 
@@ -933,7 +951,24 @@ class Solver(ThroughTransportSolver):
                                        B, X, Y, Z, self._setup_flags, self._stream())
         _lib.check(st, "tf_setup_solver")
         self._pack_sweep_codes()
+        self._groups = None
         self.vol_x = self._count.cpu().numpy().astype(np.float32) / np.float32(Y * Z)
+
+    def _sweep_groups(self):
+        """Volumes that the autotuner serves keep their codes in groups of
+        four rows as well (one byte more per voxel, packed at the first
+        launch); smaller ones run the resident sweep."""
+        voxels = self.batch_size * self.Nx * self.Ny * self.Nz
+        if self.kind != _lib.KIND_SOLVER or self._sweep_flags or voxels < autotune.MIN_VOXELS:
+            return None
+        if self._groups is None:
+            B, X, Y, Z = self.batch_size, self.Nx, self.Ny, self.Nz
+            n = B * int(self._lib.tf_sweep_groups_bytes(X, Y, Z))
+            self._groups = torch.empty(n, dtype=torch.uint8, device=self.device)
+            st = self._lib.tf_pack_sweep_groups(_lib.ptr(self._codes), _lib.ptr(self._groups), B, X, Y, Z,
+                                                self._stream())
+            _lib.check(st, "tf_pack_sweep_groups")
+        return self._groups
 
     @property
     def factor(self) -> torch.Tensor:
