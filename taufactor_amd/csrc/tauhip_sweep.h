@@ -437,6 +437,13 @@ __device__ __forceinline__ void rsweep_tile(const float* __restrict__ S, float* 
     // the wave's four rows are one group
     constexpr bool kQuad = kGroups && RPW == 4 && (2 - H) % 4 == 0 && Sh::TY % 4 == 0;
     constexpr int NQ = kGroups ? Sh::NR : 1;
+    // Every wave leaves the barrier at the same time, so loads and stores
+    // issued together at the end of a step queue up in the memory pipeline
+    // while no wave computes.  Where two planes are in flight they go between
+    // the half-sweeps of the next step instead, one plane's time later: us per
+    // half-sweep 512^3 54.0 -> 52.8, 400^3 28.7 -> 25.5, three-phase 320^3
+    // 29.0 -> 25.9.  (H = 5, one plane in flight, would wait for its loads.)
+    constexpr bool kSpread = Sh::D >= 2;
     constexpr int NG = kFaces ? Sh::NR : 1;
     constexpr int NKF = kFaceCodes ? Sh::NR : 1;
     constexpr int TY = Sh::TY, ML = Sh::ML, NR = Sh::NR, DP = Sh::D, EB = Sh::EB;
@@ -586,31 +593,34 @@ __device__ __forceinline__ void rsweep_tile(const float* __restrict__ S, float* 
     // record counts below 2^31 (a tile's planes span less than 2 GiB)
     const int rec_f = (int)(span_f + 2u * kSlackBytes);
     const int rec_c = (int)((uint32_t)(lx1 - pbase) * (uint32_t)plane_c);
-    auto issue_load = [&](int p, auto slot_c) __attribute__((always_inline)) {
+    auto issue_row = [&](int sf, int sc, auto slot_c, int j) __attribute__((always_inline)) {
         constexpr int sl = decltype(slot_c)::value;
-        const bool pok = p >= pbase && p < lx1;
-        const int sf = pok ? (p - pbase) * plane_f : rec_f, sc = pok ? (p - pbase) * plane_c : rec_c;
         if constexpr (kQuad) {
-            const u32x2_t k = __builtin_amdgcn_raw_buffer_load_b64(rC, vq[0], sc, 0);
-            KP[sl][0] = k.x;
-            KP[sl][1] = k.y;
-        } else if constexpr (kGroups) {
-#pragma unroll
-            for (int j = 0; j < RPW / 2; ++j) KP[sl][j] = __builtin_amdgcn_raw_buffer_load_b32(rC, vq[j], sc, 0);
-        }
-#pragma unroll
-        for (int j = 0; j < RPW; ++j) {
-            F[sl][j] = __builtin_amdgcn_raw_buffer_load_b64(rF, vf[j], sf, 0);
-            if constexpr (kFaces) {
-#pragma unroll
-                for (int k = 0; k < 3; ++k)
-                    G[sl][j][k] = __builtin_amdgcn_raw_buffer_load_b64(rG[k], vf[j], sf, 0);
-            } else if constexpr (kFaceCodes) {
-                KF[sl][j] = __builtin_amdgcn_raw_buffer_load_b64(rK, vf[j], sf, 0);
-            } else if constexpr (!kGroups) {
-                K[sl][j] = __builtin_amdgcn_raw_buffer_load_b16(rC, vc[j], sc, 0);
+            if (j == 0) {
+                const u32x2_t k = __builtin_amdgcn_raw_buffer_load_b64(rC, vq[0], sc, 0);
+                KP[sl][0] = k.x;
+                KP[sl][1] = k.y;
             }
+        } else if constexpr (kGroups) {
+            if (j % 2 == 0) KP[sl][j / 2] = __builtin_amdgcn_raw_buffer_load_b32(rC, vq[j / 2], sc, 0);
         }
+        F[sl][j] = __builtin_amdgcn_raw_buffer_load_b64(rF, vf[j], sf, 0);
+        if constexpr (kFaces) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) G[sl][j][k] = __builtin_amdgcn_raw_buffer_load_b64(rG[k], vf[j], sf, 0);
+        } else if constexpr (kFaceCodes) {
+            KF[sl][j] = __builtin_amdgcn_raw_buffer_load_b64(rK, vf[j], sf, 0);
+        } else if constexpr (!kGroups) {
+            K[sl][j] = __builtin_amdgcn_raw_buffer_load_b16(rC, vc[j], sc, 0);
+        }
+    };
+    auto plane_ok = [&](int p) { return p >= pbase && p < lx1; };
+    auto field_off = [&](int p) { return plane_ok(p) ? (p - pbase) * plane_f : rec_f; };
+    auto code_off = [&](int p) { return plane_ok(p) ? (p - pbase) * plane_c : rec_c; };
+    auto issue_load = [&](int p, auto slot_c) __attribute__((always_inline)) {
+        const int sf = field_off(p), sc = code_off(p);
+#pragma unroll
+        for (int j = 0; j < RPW; ++j) issue_row(sf, sc, slot_c, j);
     };
     // stores: one descriptor per plane step (based at the plane, record
     // count the plane's bytes) and one 8-byte store per row; a lane writes
@@ -631,12 +641,17 @@ __device__ __forceinline__ void rsweep_tile(const float* __restrict__ S, float* 
         const bool own = (half ? own_row[1][j] : own_row[0][j]) && zl >= z0 && zl < z1;
         so[j] = own ? ((half ? ys[1][j] : ys[0][j]) * v.sY + zl) * 4 : kOff;
     }
-    auto store_plane = [&](int q, auto slot_c) __attribute__((always_inline)) {
-        constexpr int sl = decltype(slot_c)::value;
+    auto store_rsrc = [&](int q) __attribute__((always_inline)) {
         const bool qok = q >= x0 && q < x1;
-        const rsrc_t r = make_rsrc(D + (size_t)(qok ? q : 0) * v.sX, qok ? (uint32_t)(4 * v.sX) : 0u);
+        return make_rsrc(D + (size_t)(qok ? q : 0) * v.sX, qok ? (uint32_t)(4 * v.sX) : 0u);
+    };
+    auto store_row = [&](rsrc_t r, auto slot_c, int j) __attribute__((always_inline)) {
+        __builtin_amdgcn_raw_buffer_store_b64(F[decltype(slot_c)::value][j], r, so[j], 0, kStoreNT);
+    };
+    auto store_plane = [&](int q, auto slot_c) __attribute__((always_inline)) {
+        const rsrc_t r = store_rsrc(q);
 #pragma unroll
-        for (int j = 0; j < RPW; ++j) __builtin_amdgcn_raw_buffer_store_b64(F[sl][j], r, so[j], 0, kStoreNT);
+        for (int j = 0; j < RPW; ++j) store_row(r, slot_c, j);
     };
 
     // ---- per-tile bounds of each half-sweep (planes only: rows and z are
@@ -925,7 +940,7 @@ __device__ __forceinline__ void rsweep_tile(const float* __restrict__ S, float* 
 
         // planes S0-1 .. S0+1+DP in flight; plane S0's edges published as
         // "step S0-1" for the first half-sweep
-        static_for<0, DP + 3>([&](auto i_c) __attribute__((always_inline)) {
+        static_for<0, kSpread ? DP + 2 : DP + 3>([&](auto i_c) __attribute__((always_inline)) {
             constexpr int i = decltype(i_c)::value;
             issue_load(S0 - 1 + i, ic<i>{});
         });
@@ -938,15 +953,30 @@ __device__ __forceinline__ void rsweep_tile(const float* __restrict__ S, float* 
             static_for<0, NR>([&](auto u_c) __attribute__((always_inline)) {
                 constexpr int u = decltype(u_c)::value;
                 const int s = s0 + u;
+                // kSpread: the plane that the step before finished and the load
+                // into the slot that it freed, a row at a time between the
+                // half-sweeps of this step
+                const rsrc_t rS = store_rsrc(s - H);
+                const int sf = field_off(s + 1 + DP), sc = code_off(s + 1 + DP);
                 static_for<0, H>([&](auto h_c) __attribute__((always_inline)) {
                     constexpr int h = decltype(h_c)::value;
                     stage(h_c, u_c, s - h, chk_c);
                     if constexpr (h + 1 < H) publish(h + 1, u, ic<((u - h + 1) % NR + NR) % NR>{});
+                    if constexpr (kSpread) {
+                        // this stage's share of the 2 RPW rows to move
+                        static_for<0, RPW>([&](auto j_c) __attribute__((always_inline)) {
+                            constexpr int j = decltype(j_c)::value;
+                            if constexpr (2 * j * H / (2 * RPW) == h) store_row(rS, ic<(u - H + 1 + NR) % NR>{}, j);
+                            if constexpr ((2 * j + 1) * H / (2 * RPW) == h) issue_row(sf, sc, ic<(u - H + NR) % NR>{}, j);
+                        });
+                    }
                 });
                 publish(0, u, ic<(u + 2) % NR>{});
                 publish_faces(ic<(u + 2) % NR>{});
-                store_plane(s - (H - 1), ic<((u - H + 2) % NR + NR) % NR>{});
-                issue_load(s + 2 + DP, ic<((u - H + 1) % NR + NR) % NR>{});
+                if constexpr (!kSpread) {
+                    store_plane(s - (H - 1), ic<((u - H + 2) % NR + NR) % NR>{});
+                    issue_load(s + 2 + DP, ic<((u - H + 1) % NR + NR) % NR>{});
+                }
                 __syncthreads();
             });
         };
@@ -975,6 +1005,7 @@ __device__ __forceinline__ void rsweep_tile(const float* __restrict__ S, float* 
             for (; s0 >= s_lo && s0 <= s_hi; s0 += NR) block(s0, std::false_type{});
         }
         for (; s0 <= S1; s0 += NR) block(s0, std::true_type{});
+        if constexpr (kSpread) store_plane(s0 - H, ic<(NR - H + 1) % NR>{});  // of the last step, s0 - 1
     };
     body(ic<AC>{});
 }
