@@ -8,7 +8,7 @@ and keeps the one with the lowest time per reference iteration:
 * plain solvers (Solver, MultiPhaseSolver, FieldSolver): a few launches of
   each candidate on scratch copies of the current field, so the solver's
   state is untouched;
-* BatchSolver: a few passes of each candidate over the whole packed batch,
+* BatchSolver (large batches): a few passes of each candidate over the whole packed batch,
   after which the batch is re-packed (a depth that does not divide 100 ends
   each period with one shorter pass, not timed here).
 
@@ -58,6 +58,27 @@ def small_volume_default(voxels: int):
     if voxels < 3 * (1 << 20):
         return (4, (8, 2, 0))
     return (None, None)
+
+
+def batch_default(voxels: int):
+    """(H, tile) for an uneven batch of fewer than 2^26 voxels in all; (None,
+    None) leaves it to tune_batch.  A pass is at least one tile's stream of
+    tx + 2 (H - 1) planes long, and most passes of a batch run when few
+    volumes are left: short x tiles serve them, where the tuner, which times
+    passes over every volume, prefers long ones.  Whole solves on MI355X, ms,
+    against 4 x (8 or 16 waves x 2 rows, x tile 64), the tuner's choice or the
+    default before: 12 volumes of edge 20 to 60 5.9 -> 2.7 (8 x 2, tile 16),
+    6 of 40 to 128 7.8 -> 4.0 (16 x 2, tile 16; tile 32 5.6), 24 of 96 to 128
+    16.1 -> 14.3 (tile 32; tile 16 13.9), 48 of 64 to 128 17.2 -> 16.0 (tile
+    16 17.3).  At 32 of 96 to 224 (112 M voxels) tile 64 is the best again:
+    67.7 against 72.8 and 83."""
+    if voxels < 1 << 21:
+        return 5, (8, 2, 16)
+    if voxels < 3 << 23:
+        return 5, (16, 2, 16)
+    if voxels < 1 << 26:
+        return 5, (16, 2, 32)
+    return None, None
 
 
 def _candidates(space, fixed_h, fixed_tile):

@@ -250,13 +250,15 @@ class BatchSolver:
         return src_b
 
     def _launch_config(self):
-        """(H, tile): explicit settings win, then the autotuner for batches of
-        at least autotune.MIN_VOXELS voxels, then H = 4 and the default tile."""
+        """(H, tile): explicit settings win, then autotune.batch_default or,
+        for the batches it leaves open, the autotuner."""
         H, tile = self.half_sweeps_per_pass, self.tile
         if H is not None and tile is not None:
             return int(H), tuple(tile)
         aH, atile = None, None
-        if self.autotune and sum(X * Y * Z for X, Y, Z in self.shapes) >= autotune.MIN_VOXELS:
+        if self.autotune and H is None and tile is None:
+            aH, atile = autotune.batch_default(sum(X * Y * Z for X, Y, Z in self.shapes))
+        if self.autotune and aH is None and sum(X * Y * Z for X, Y, Z in self.shapes) >= autotune.MIN_VOXELS:
             aH, atile = autotune.tune_batch(self, H, tile)
         H = int(H) if H is not None else (aH or 4)
         tile = tuple(tile) if tile is not None else atile
