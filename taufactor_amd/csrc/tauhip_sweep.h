@@ -439,10 +439,10 @@ __device__ __forceinline__ void rsweep_tile(const float* __restrict__ S, float* 
     constexpr int NQ = kGroups ? Sh::NR : 1;
     // Every wave leaves the barrier at the same time, so loads and stores
     // issued together at the end of a step queue up in the memory pipeline
-    // while no wave computes.  Where two planes are in flight they go between
-    // the half-sweeps of the next step instead, one plane's time later: us per
-    // half-sweep 512^3 54.0 -> 52.8, 400^3 28.7 -> 25.5, three-phase 320^3
-    // 29.0 -> 25.9.  (H = 5, one plane in flight, would wait for its loads.)
+    // while no wave computes.  The stores go between the half-sweeps of the
+    // next step instead, and where two planes are in flight the loads too (at
+    // H = 5, with one, they would be waited for): us per half-sweep 512^3
+    // 54.0 -> 52.8, 400^3 28.7 -> 25.5, three-phase 320^3 29.0 -> 25.9.
     constexpr bool kSpread = Sh::D >= 2;
     constexpr int NG = kFaces ? Sh::NR : 1;
     constexpr int NKF = kFaceCodes ? Sh::NR : 1;
@@ -647,11 +647,6 @@ __device__ __forceinline__ void rsweep_tile(const float* __restrict__ S, float* 
     };
     auto store_row = [&](rsrc_t r, auto slot_c, int j) __attribute__((always_inline)) {
         __builtin_amdgcn_raw_buffer_store_b64(F[decltype(slot_c)::value][j], r, so[j], 0, kStoreNT);
-    };
-    auto store_plane = [&](int q, auto slot_c) __attribute__((always_inline)) {
-        const rsrc_t r = store_rsrc(q);
-#pragma unroll
-        for (int j = 0; j < RPW; ++j) store_row(r, slot_c, j);
     };
 
     // ---- per-tile bounds of each half-sweep (planes only: rows and z are
@@ -953,30 +948,26 @@ __device__ __forceinline__ void rsweep_tile(const float* __restrict__ S, float* 
             static_for<0, NR>([&](auto u_c) __attribute__((always_inline)) {
                 constexpr int u = decltype(u_c)::value;
                 const int s = s0 + u;
-                // kSpread: the plane that the step before finished and the load
-                // into the slot that it freed, a row at a time between the
-                // half-sweeps of this step
+                // the plane that the step before finished and (kSpread) the
+                // load into the slot that it freed, a row at a time between
+                // the half-sweeps of this step
                 const rsrc_t rS = store_rsrc(s - H);
                 const int sf = field_off(s + 1 + DP), sc = code_off(s + 1 + DP);
                 static_for<0, H>([&](auto h_c) __attribute__((always_inline)) {
                     constexpr int h = decltype(h_c)::value;
                     stage(h_c, u_c, s - h, chk_c);
                     if constexpr (h + 1 < H) publish(h + 1, u, ic<((u - h + 1) % NR + NR) % NR>{});
-                    if constexpr (kSpread) {
-                        // this stage's share of the 2 RPW rows to move
-                        static_for<0, RPW>([&](auto j_c) __attribute__((always_inline)) {
-                            constexpr int j = decltype(j_c)::value;
-                            if constexpr (2 * j * H / (2 * RPW) == h) store_row(rS, ic<(u - H + 1 + NR) % NR>{}, j);
-                            if constexpr ((2 * j + 1) * H / (2 * RPW) == h) issue_row(sf, sc, ic<(u - H + NR) % NR>{}, j);
-                        });
-                    }
+                    // this stage's share of the rows to move
+                    static_for<0, RPW>([&](auto j_c) __attribute__((always_inline)) {
+                        constexpr int j = decltype(j_c)::value;
+                        if constexpr (j * H / RPW == h) store_row(rS, ic<(u - H + 1 + NR) % NR>{}, j);
+                        if constexpr (kSpread && (2 * j + 1) * H / (2 * RPW) == h)
+                            issue_row(sf, sc, ic<(u - H + NR) % NR>{}, j);
+                    });
                 });
                 publish(0, u, ic<(u + 2) % NR>{});
                 publish_faces(ic<(u + 2) % NR>{});
-                if constexpr (!kSpread) {
-                    store_plane(s - (H - 1), ic<((u - H + 2) % NR + NR) % NR>{});
-                    issue_load(s + 2 + DP, ic<((u - H + 1) % NR + NR) % NR>{});
-                }
+                if constexpr (!kSpread) issue_load(s + 2 + DP, ic<((u - H + 1) % NR + NR) % NR>{});
                 __syncthreads();
             });
         };
@@ -1005,7 +996,10 @@ __device__ __forceinline__ void rsweep_tile(const float* __restrict__ S, float* 
             for (; s0 >= s_lo && s0 <= s_hi; s0 += NR) block(s0, std::false_type{});
         }
         for (; s0 <= S1; s0 += NR) block(s0, std::true_type{});
-        if constexpr (kSpread) store_plane(s0 - H, ic<(NR - H + 1) % NR>{});  // of the last step, s0 - 1
+        // the plane of the last step, s0 - 1
+        const rsrc_t rS = store_rsrc(s0 - H);
+#pragma unroll
+        for (int j = 0; j < RPW; ++j) store_row(rS, ic<(NR - H + 1) % NR>{}, j);
     };
     body(ic<AC>{});
 }
