@@ -66,9 +66,9 @@ METRIC = "GVoxel-updates/s + % HBM roofline; solves/s batched vs plain @ D_eff r
 HBM_PEAK_GBS = 8000.0
 BYTES_PER_UPDATE = {"code": 9, "field": 12}
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "sweep_traffic.json")
-# the compilation unit of each workload's sweep kernel (its traffic entry is
+# the compilation unit of each kind's sweep kernel (its traffic entry is
 # keyed to the hash of that unit, the shared sweep header and the flags)
-SWEEP_UNITS = {"C2": "sweep_solver.hip", "C4": "sweep_mpfaces.hip", "C5": "sweep_field.hip"}
+SWEEP_UNITS = {"Solver": "sweep_solver.hip", "MultiPhaseFaces": "sweep_mpfaces.hip", "Field": "sweep_field.hip"}
 
 
 def log(msg: str) -> None:
@@ -98,15 +98,35 @@ def roofline(kind: str, nvox: int, H: int, mean_launch_s: float, kernel: str) ->
             "mean_launch_ms": round(mean_launch_s * 1e3, 4), "traffic": None}
 
 
-def attach_traffic(rl: dict, workload: str, H: int, tile, mean_launch_s: float) -> None:
+def sweep_kernel(s, kind: str, H: int, tile):
+    """(half-sweeps per timed launch, kernel, its compilation unit) of the
+    sweep that solver s ran: a resident launch counts its half-sweeps, and
+    large Solver volumes read their codes in groups."""
+    if s._resident:
+        return 1, f"k_resident<{kind}>", None
+    if s._groups is not None and s._launch_operands(H, _tile(tile))[0] != s.kind:
+        return H, f"k_sweep<{H}, {kind}Groups, {tile[0]}, {tile[1]}>", "sweep_solver_groups.hip"
+    return H, f"k_sweep<{H}, {kind}, {tile[0]}, {tile[1]}>", SWEEP_UNITS.get(kind)
+
+
+def _tile(tile):
+    from taufactor_amd import _lib
+
+    return _lib.Tile(*tile)
+
+
+def attach_traffic(rl: dict, workload: str, H: int, tile, mean_launch_s: float, unit) -> None:
     """Measured HBM bytes per launch from the committed summary of this
     kernel build, when there is one for this workload, depth and tile."""
+    if unit is None:
+        rl["traffic_note"] = "no traffic summary for this kernel"
+        return
     if not os.path.exists(TRAFFIC_FILE):
         rl["traffic_note"] = "no traffic summary committed"
         return
     with open(TRAFFIC_FILE) as f:
         entries = json.load(f)
-    src = sweep_source_sha256(SWEEP_UNITS[workload])
+    src = sweep_source_sha256(unit)
     for t in entries:
         if (t.get("workload") == workload and t.get("half_sweeps_per_pass") == H and t.get("tile") == list(tile)
                 and t.get("source_sha256") == src):
@@ -187,8 +207,9 @@ def run_solver512(args, dev):
     s._launch_events = None
     nvox = img.size
     gvus = nvox * sum(iters) / 2 / elapsed / 1e9
-    rl = roofline("code", nvox, H, mean_s, f"k_sweep<{H}, Solver, {rtile[0]}, {rtile[1]}>")
-    attach_traffic(rl, "C2", H, rtile, mean_s)
+    h, kernel, unit = sweep_kernel(s, "Solver", H, rtile)
+    rl = roofline("code", nvox, h, mean_s, kernel)
+    attach_traffic(rl, "C2", H, rtile, mean_s, unit)
     log(f"{args.steps} solves, iterations {iters}, {elapsed:.3f} s -> {gvus:.1f} GVoxel-updates/s; "
         f"sweep kernel {mean_s * 1e3:.4f} ms -> effective frac {rl['frac']}, dram frac {rl.get('dram_frac')}")
     out = {
@@ -327,10 +348,9 @@ def run_multiphase320(dev, launch=None) -> dict:
     fwd = {"iterations": s.iter, "tau": float(s.tau[0]), "D_eff": float(s.D_eff[0]), "ms": round(t_fwd * 1e3, 3),
            "GVoxel_updates_per_s": round(gvus, 3)}
     faces = s._faces is not None
-    rl = roofline("code", nvox, H, mean_s,
-                  f"k_sweep<{H}, {'MultiPhaseFaces' if faces else 'MultiPhase'}, {tile[0]}, {tile[1]}>")
-    if faces:
-        attach_traffic(rl, "C4", H, tile, mean_s)
+    h, kernel, unit = sweep_kernel(s, "MultiPhaseFaces" if faces else "MultiPhase", H, tile)
+    rl = roofline("code", nvox, h, mean_s, kernel)
+    attach_traffic(rl, "C4", H, tile, mean_s, unit)
     del s
     s, g, t_f, t_b = _grad_timing(lambda: _with_launch(tau.MultiPhaseSolver(img, dict(Ds), device=dev), launch),
                                   1e-3, lambda x: x.grad_D_eff())
@@ -379,8 +399,9 @@ def run_field128x64(dev, launch=None) -> dict:
     gvus = nvox * s.iter / 2 / t_fwd / 1e9
     fwd = {"iterations": s.iter, "D_eff_mean": float(s.D_eff.mean()), "ms": round(t_fwd * 1e3, 3),
            "GVoxel_updates_per_s": round(gvus, 3)}
-    rl = roofline("field", nvox, H, mean_s, f"k_sweep<{H}, Field, {tile[0]}, {tile[1]}>")
-    attach_traffic(rl, "C5", H, tile, mean_s)
+    h, kernel, unit = sweep_kernel(s, "Field", H, tile)
+    rl = roofline("field", nvox, h, mean_s, kernel)
+    attach_traffic(rl, "C5", H, tile, mean_s, unit)
     del s
     s, g, t_f, t_b = _grad_timing(lambda: _with_launch(tau.FieldSolver(kt, device=dev), launch), 1e-4,
                                   lambda x: x.grad_D_eff())

@@ -85,7 +85,8 @@ class SORSolver(ABC):
         self._cur = 0
         self._spare = None  # third buffer: more sweeps ahead of a check
         self._checked = None  # (buffers, index) of the checked field
-        self._launch_events = None  # list -> (start, end, n_launches) per _advance
+        # list -> (start, end, launches, or half-sweeps of a resident launch) per _advance
+        self._launch_events = None
         self._codes = None
         self._sweep_codes = None
         self._groups = None  # see Solver._sweep_groups
@@ -703,7 +704,7 @@ class _ResidentSweep:
         _lib.check(st, "tf_sweep_resident")
         if ev is not None:
             t1.record()
-            ev.append((t0, t1, 1))
+            ev.append((t0, t1, n))
         self.log.append((self.count, src, it))
         s._cur = 1 - s._cur
         return True
