@@ -8,9 +8,9 @@ and keeps the one with the lowest time per reference iteration:
 * plain solvers (Solver, MultiPhaseSolver, FieldSolver): a few launches of
   each candidate on scratch copies of the current field, so the solver's
   state is untouched;
-* BatchSolver (large batches): a few passes of each candidate over the whole packed batch,
-  after which the batch is re-packed (a depth that does not divide 100 ends
-  each period with one shorter pass, not timed here).
+* BatchSolver (large batches): a few passes of each candidate over the whole
+  packed batch, after which the batch is re-packed (a depth that does not
+  divide 100 ends each period with one shorter pass, not timed here).
 
 Results are cached per (kind, batch, shape) for the life of the process.
 Volumes below MIN_VOXELS are not tuned: the defaults (H = 4, library tile)
@@ -26,6 +26,10 @@ MIN_VOXELS = 1 << 23
 # even, so that a candidate with an odd H is timed on as many launches of
 # each starting colour
 TIMED_LAUNCHES = 6
+# of a plain solver's first look at each depth and shape, and before it
+FIRST_LAUNCHES = 2
+WARM_LAUNCHES = 4
+NEAR = 1.15  # of the fastest there: timed again, with every x tile
 
 # (H values, workgroup shapes, x-tile lengths), in order of preference: the
 # first candidate within TIE of the fastest wins, which keeps the choice
@@ -128,7 +132,9 @@ def tune_solver(s, fixed_h=None, fixed_tile=None):
     candidates = _candidates(space, fixed_h, fixed_tile)
     if fixed_tile is None and s._sweep_groups() is not None:
         candidates += [c for c in _candidates(GROUP_SPACE, fixed_h, None) if c[0] in _lib.GROUP_DEPTHS]
-    for H, tile in candidates:
+
+    def timed(H, tile, n):
+        """ms per half-sweep of n launches, None if one is refused."""
         kind, codes, hm, n_table, t = s._launch_operands(H, _lib.Tile(*tile))
         bufs = [src, dst]
         state = {"i": 0}
@@ -142,9 +148,27 @@ def tune_solver(s, fixed_h=None, fixed_tile=None):
             return lib.tf_sweep(_lib.ptr(bufs[i & 1]), _lib.ptr(bufs[1 - (i & 1)]), codes, hm,
                                 n_table, kind, B, X, Y, Z, s._w32, (i * H) & 1, H, t, stream)
 
-        ms = _time(launch, TIMED_LAUNCHES)
-        if ms is not None:
-            timings.append((ms / H, H, tile))
+        ms = _time(launch, n)
+        return None if ms is None else ms / H
+
+    # a first look at every depth and shape, with its first x tile; the other
+    # x tiles and the longer timing only for those near the fastest (on a new
+    # 512^3 volume every candidate in full took 137 ms, this takes 40; 400^3 69
+    # and 13, three-phase 320^3 62 and 28, with the same choices).  The clocks rise
+    # over the first launches, which would count against whatever comes first.
+    for _ in range(WARM_LAUNCHES):
+        if timed(*candidates[0], 1) is None:
+            break
+    first = {}
+    for H, tile in candidates:
+        if (H, tile[:2]) not in first:
+            first[H, tile[:2]] = timed(H, tile, FIRST_LAUNCHES)
+    limit = min((t for t in first.values() if t is not None), default=0.0) * NEAR
+    for H, tile in candidates:
+        if first[H, tile[:2]] is not None and first[H, tile[:2]] <= limit:
+            t = timed(H, tile, TIMED_LAUNCHES)
+            if t is not None:
+                timings.append((t, H, tile))
     del src, dst
     last_timings[:] = timings
     result = _pick(timings)
