@@ -644,9 +644,9 @@ class _ResidentSweep:
         plan = _lib.Resident()
         cus = torch.cuda.get_device_properties(s.device).multi_processor_count
         # the kinds with face conductances also run batches in several
-        # launches (groups of equally many volumes): 0.7 ns per voxel and
+        # launches (groups of equally many volumes): 0.7 ps per voxel and
         # half-sweep of 4 x 128^3 against 1.6 streaming; the others stream a
-        # batch that does not fit at once, at 0.5 to 0.7 ns
+        # batch that does not fit at once, at 0.5 to 0.7 ps
         B = s.batch_size
         most = B if kind in (_lib.KIND_FIELD, _lib.KIND_MULTIPHASE_FACES) else 1
         for groups in range(1, most + 1):
