@@ -412,7 +412,9 @@ def run_field128x64(dev, launch=None) -> dict:
         "workload": "64 volumes of 128^3, k = sigmoid(4 z), z standardised smoothed noise sigma 3 "
                     "(all volumes stop together, the reference's batch semantics)",
         "forward_conv_1e-2": fwd, "roofline": rl,
-        "half_sweeps_per_pass": H, "tile": list(tile), "tiles_per_launch": n_tiles,
+        # (the streaming sweep's; a resident launch runs until the next check)
+        "half_sweeps_per_pass": H if unit else None, "tile": list(tile) if unit else None,
+        "tiles_per_launch": n_tiles if unit else None,
         "gradient": {"forward_conv_crit": 1e-4, "forward_iterations": s.iter, "forward_converged": bool(s.converged),
                      "forward_ms": round(t_f * 1e3, 3),
                      "backward_ms": round(t_b * 1e3, 3), "backward_over_forward": round(t_b / t_f, 5),
