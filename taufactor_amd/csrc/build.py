@@ -14,13 +14,14 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.dirname(HERE)
 ROOT = os.path.dirname(PKG)
-# the C-ABI and non-sweep kernels, then one unit per sweep kind (compiled in
-# parallel: the sweep templates dominate the build)
-SOURCES = ["tauhip.hip", "sweep_solver.hip", "sweep_solver_groups.hip", "sweep_multiphase.hip",
-           "sweep_mpfaces.hip", "sweep_field.hip",
-           "sweep_anisotropic.hip", "sweep_electrode.hip", "sweep_batch.hip",
-           "resident_solver.hip", "resident_periodic.hip", "resident_anisotropic.hip", "resident_electrode.hip",
-           "resident_field.hip", "resident_mpfaces.hip"]
+# the C-ABI and non-sweep kernels (tauhip.hip), then one unit or two per sweep
+# kind, the longest to compile first (in parallel: the sweep templates dominate
+# the build)
+SOURCES = ["sweep_batch_deep.hip", "sweep_solver_deep.hip", "sweep_batch.hip", "sweep_solver.hip",
+           "sweep_multiphase.hip", "sweep_mpfaces.hip", "sweep_field.hip", "resident_electrode.hip",
+           "resident_solver.hip", "resident_periodic.hip", "sweep_solver_groups.hip", "resident_anisotropic.hip",
+           "resident_mpfaces.hip", "sweep_anisotropic.hip", "sweep_electrode.hip", "resident_field.hip",
+           "tauhip.hip"]
 INCLUDE = os.path.join(ROOT, "include")
 OUT = os.path.join(PKG, "libtauhip.so")
 OBJ_DIR = os.path.join(HERE, "_build")
