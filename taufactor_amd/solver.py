@@ -375,6 +375,7 @@ class SORSolver(ABC):
         second writes that one, which takes the checked field's place in the
         pair, so no sweep writes the checked field and, if the solve stops
         there, _drop_ahead returns to it unchanged."""
+        self._checked = None  # (a decision before this one may have kept its own)
         room = self._ahead_room(n_next)
         if room <= 0:
             return

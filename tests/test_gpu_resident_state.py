@@ -1,0 +1,32 @@
+"""GPU: solvers that change between resident and streaming launches, or stop
+between checks, against the oracle's field."""
+import numpy as np
+import pytest
+
+import taufactor_amd as tau
+from oracle.restate import OracleMultiPhaseSolver, OracleSolver
+
+pytestmark = pytest.mark.gpu
+
+
+def _labels(shape, n, seed):
+    return np.random.default_rng(seed).integers(0, n, size=shape).astype(np.uint8)
+
+
+D3 = {0: 0.0, 1: 1.0, 2: 0.1}
+
+
+@pytest.mark.parametrize("cls,ocls,n,extra", [(tau.Solver, OracleSolver, 2, ()),
+                                              (tau.MultiPhaseSolver, OracleMultiPhaseSolver, 3, (D3,))])
+def test_back_from_a_hand_set_depth(cls, ocls, n, extra):
+    """Streaming up to a check, then the default: the converged field is that
+    of the last check."""
+    img = _labels((22, 20, 21), n, 3)
+    img[:, 4:9, 5:12] = 1
+    s = cls(img, *(dict(e) for e in extra))
+    s.half_sweeps_per_pass = 4
+    s.solve(iter_limit=200, verbose=False, conv_crit=0.0)
+    s.half_sweeps_per_pass = None
+    s.solve(verbose=False)
+    assert s.converged and s.iter > 200 and s._resident
+    assert np.array_equal(s.field.cpu().numpy(), ocls(img, *(dict(e) for e in extra)).run(s.iter).field.numpy())

@@ -1,0 +1,187 @@
+"""CPU: the host logic of the resident and streaming launches (which buffer a
+launch reads and writes, launches ahead of a check that are dropped, launches
+whose waits ran out) on a stand-in for the device.
+
+The stand-in's field holds, in every interior voxel, the number of iterations
+behind it, and in its x ghosts the boundary value it was given; a launch
+requires its source to hold the iteration it starts from.  As on the device, a
+lost resident launch stores its number in the status and leaves dst void, and
+later resident launches write nothing until the status is cleared."""
+import contextlib
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import taufactor_amd as tau
+from taufactor_amd import _lib, solver as solver_module
+
+VOID = -1e6  # what a lost launch leaves
+X = Y = Z = 4
+
+
+class Device:
+    """The library entry points that a solve calls, on host memory."""
+
+    def __init__(self):
+        self.lost = set()  # resident launches (counted from 1) whose waits run out
+        self.launches = 0
+        self.boundary = 0.5
+
+    def _view(self, p, dtype, n):
+        return np.ctypeslib.as_array((dtype * n).from_address(p))
+
+    def _field(self, p):
+        return self._view(p, ctypes.c_float, (X + 2) * (Y + 2) * (Z + 2)).reshape(X + 2, Y + 2, Z + 2)
+
+    def _run(self, src, dst, n, colour):
+        s, d = self._field(src), self._field(dst)
+        it = s[1, 1, 1]
+        assert np.all(s[1:-1, 1:-1, 1:-1] == it) and it >= 0, "a void field was read"
+        assert np.all(s[[0, -1]] == self.boundary), "a field with other boundary values was read"
+        assert int(it) & 1 == colour, f"iteration {it} read for a launch of colour {colour}"
+        d[1:-1, 1:-1, 1:-1] = it + n
+
+    def tf_sweep(self, src, dst, codes, hm, n_table, kind, B, nx, ny, nz, w, colour, h, tile, stream):
+        self._run(src, dst, h, colour)
+        return 0
+
+    def tf_resident_plan(self, kind, B, nx, ny, nz, cus, plan):
+        plan._obj.mail_bytes = 64
+        return 1
+
+    def tf_sweep_resident(self, src, dst, codes, table, n_table, kind, B, nx, ny, nz, w, colour, n, plan, section,
+                          mail, mail_bytes, tag, status, launch_id, spin, stream):
+        st = self._view(status, ctypes.c_int32, 1)
+        self.launches += 1
+        if st[0]:
+            return 0
+        if self.launches in self.lost:
+            st[0] = launch_id
+            self._field(dst)[1:-1, 1:-1, 1:-1] = VOID
+        else:
+            self._run(src, dst, n, colour)
+        return 0
+
+    def tf_wrap_ghosts_from(self, *args):
+        return 0
+
+    def tf_hbm_copy(self, src, dst, n, stream):
+        ctypes.memmove(dst, src, n)
+        return 0
+
+    def tf_layer_sums_ws(self, field, codes, hm, n_classes, kind, B, nx, ny, nz, flux, conc, ws, n_ws, stream):
+        # the value of the field that is checked
+        self._view(flux, ctypes.c_double, 1)[0] = self._field(field)[1, 1, 1]
+        return 0
+
+
+class _Event:
+    def __init__(self, *a, **k):
+        pass
+
+    def record(self, *a):
+        pass
+
+    def synchronize(self):
+        pass
+
+
+class _Stream:
+    cuda_stream = 7
+
+    def wait_event(self, e):
+        pass
+
+    def record_event(self, e=None):
+        return e or _Event()
+
+    def __eq__(self, other):
+        return self.cuda_stream == other.cuda_stream
+
+    __hash__ = None
+
+
+@pytest.fixture
+def device(monkeypatch):
+    for name, f in {"device": lambda d: contextlib.nullcontext(), "synchronize": lambda d=None: None,
+                    "Event": _Event, "current_stream": lambda d=None: _Stream(),
+                    "get_device_properties": lambda d: type("P", (), {"multi_processor_count": 256})}.items():
+        monkeypatch.setattr(torch.cuda, name, f)
+    monkeypatch.setattr(solver_module, "_resident_turn", {})
+    monkeypatch.setattr(_lib, "stream_handle", lambda d: _Stream.cuda_stream)
+    return Device()
+
+
+def make(cls, device, spare=True):
+    """A solver of the class on the stand-in, its fields at iteration 0."""
+
+    class Stub(cls):
+        stop = None  # iteration at which the check finds convergence
+
+        def _launch_operands(self, H, tile):
+            return self.kind | self._sweep_flags, 0, None, 0, tile
+
+        def compute_metrics(self):
+            flux, _ = self._layer_sums()
+            assert self._sums_host[0] == self.iter, "another field was checked"
+            done = self.stop is not None and self.iter >= self.stop
+            return np.ones(1), np.full(1, 0.0 if done else 1.0)
+
+        def _end_simulation(self, iterations, verbose):
+            pass
+
+    s = object.__new__(Stub)
+    s.batch_size, s.Nx, s.Ny, s.Nz = 1, X, Y, Z
+    s.device = torch.device("cpu")
+    s._lib = device
+    s._w32, s.omega = 1.5, 1.5
+    s.half_sweeps_per_pass = s.tile = s._auto_cfg = None
+    s.autotune = True
+    shape = (1, X + 2, Y + 2, Z + 2)
+    s._fields = [_lib.slack_buffer(shape, torch.float32, s.device) for _ in range(2)]
+    for f in s._fields:
+        f[:, [0, -1]] = device.boundary
+    s._field_init = _lib.slack_buffer(shape, torch.float32, s.device)
+    s._copy_field(s._fields[0], s._field_init)
+    s._spare = None
+    if spare and s._zero_yz_ghosts:
+        s._spare = _lib.slack_buffer(shape, torch.float32, s.device)
+        s._copy_field(s._field_init, s._spare)
+    s._codes = s._sweep_codes = torch.zeros(4096, dtype=torch.uint8)
+    s._groups = s._hm_lut = s._launch_events = s._checked = None
+    s._n_classes = 0
+    s._sums = torch.zeros(2 * X + 1, dtype=torch.float64)
+    s._sums_host = torch.zeros(2 * X + 1, dtype=torch.float64)
+    s._sums_ws = torch.zeros(1, dtype=torch.float64)
+    s._resident = s._sums_ready = None
+    s._cur = s._ahead = s.iter = s.old_tau = 0
+    s.converged = False
+    s.tau = s.tau_x = s.D_eff = None
+    return s
+
+
+def holds(s, device):
+    """The solver's field is that of its iteration, with its boundary."""
+    f = s.field[0].numpy()
+    assert np.all(f[1:-1, 1:-1, 1:-1] == s.iter), (f[1, 1, 1], s.iter)
+    assert np.all(f[[0, -1]] == device.boundary)
+
+
+def run(s, limit, stop=None):
+    s.stop, s.converged = stop, False
+    s.solve(iter_limit=limit, verbose=False)
+
+
+def test_back_from_a_hand_set_depth(device):
+    """A solve that streams (depth set by hand) and ends on a check, then the
+    default again: a resident solve that converges ends on its own field, not
+    on one that the streaming solve's last decision kept."""
+    s = make(tau.Solver, device)
+    s.half_sweeps_per_pass = 4
+    run(s, 200)
+    s.half_sweeps_per_pass = None
+    run(s, 10000, stop=400)
+    assert s.converged and s.iter == 400
+    holds(s, device)
