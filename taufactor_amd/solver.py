@@ -1492,7 +1492,8 @@ class _PeriodicYZ:
         if r and r.log:
             if r.third is None:
                 r.third = _lib.slack_buffer(tuple(self._field_init.shape), torch.float32, self.device)
-                self._copy_field(self._field_init, r.third)
+                # (the x ghosts may have been set since the set-up)
+                self._copy_field(self._fields[self._cur], r.third)
             k = 1 - self._cur
             self._fields[k], r.third = r.third, self._fields[k]
         SORSolver._advance(self, 1, resident=False)

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 import taufactor_amd as tau
-from oracle.restate import OracleMultiPhaseSolver, OracleSolver
+from oracle.restate import OracleMultiPhaseSolver, OraclePeriodicSolver, OracleSolver
 
 pytestmark = pytest.mark.gpu
 
@@ -30,3 +30,18 @@ def test_back_from_a_hand_set_depth(cls, ocls, n, extra):
     s.solve(verbose=False)
     assert s.converged and s.iter > 200 and s._resident
     assert np.array_equal(s.field.cpu().numpy(), ocls(img, *(dict(e) for e in extra)).run(s.iter).field.numpy())
+
+
+def test_periodic_with_other_electrode_values():
+    """The x ghosts of a field that is set before the first solve hold in
+    every buffer of a resident periodic solve."""
+    img = (np.random.default_rng(6).random((18, 20, 22)) < 0.7).astype(np.uint8)
+    s, o = tau.PeriodicSolver(img), OraclePeriodicSolver(img)
+    f = o.field.clone()
+    f[:, 0], f[:, -1] = f[:, 0] * 0.5, f[:, -1] * 2
+    o.field = f.clone()
+    s.field = f.to(s.device)
+    for n in (230, 170):
+        o.run(n)
+        s.solve(iter_limit=s.iter + n, verbose=False, conv_crit=0.0)
+        assert s._resident and np.array_equal(s.field.cpu().numpy(), o.field.numpy())

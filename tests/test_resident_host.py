@@ -185,3 +185,15 @@ def test_back_from_a_hand_set_depth(device):
     run(s, 10000, stop=400)
     assert s.converged and s.iter == 400
     holds(s, device)
+
+
+def test_boundary_set_before_the_third_buffer(device):
+    """A field with other x ghosts, set before a periodic solver's first
+    launch, holds in the third buffer too."""
+    s = make(tau.PeriodicSolver, device)
+    f = s.field.clone()
+    f[:, [0, -1]] = device.boundary = 0.25
+    s.field = f
+    run(s, 330)
+    assert s._resident.third is not None
+    holds(s, device)
