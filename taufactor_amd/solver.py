@@ -331,10 +331,13 @@ class SORSolver(ABC):
         """Run n_half reference iterations (half-sweeps) on the device; the
         first self._ahead of them were launched ahead of the last check.
         resident False: with streaming launches in any case."""
+        resident = resident and self._resident_sweep()
+        if not resident and self._resident and any(src is f for _, src, _ in self._resident.log for f in self._fields):
+            self._settle()  # a field that a lost launch would be repeated from must not be written
         done, self._ahead = self._ahead, 0
         it = self.iter + done
         n_half -= done
-        if n_half > 0 and resident and self._resident_sweep() and self._resident.launch(self, n_half, it):
+        if n_half > 0 and resident and self._resident.launch(self, n_half, it):
             return
         per, tile = self._sweep_args()
         # timing (bench.py): HIP events on the launch stream around the
@@ -573,6 +576,7 @@ class SORSolver(ABC):
                     if self.converged:
                         self._drop_ahead()
             torch.cuda.synchronize(self.device)
+            self._settle()
             self.walltime = timer() - start
             self._end_simulation(self.iter, verbose)
             if self.tau_x is None:
@@ -1505,10 +1509,10 @@ class _PeriodicYZ:
                 if n_half > 1:
                     SORSolver._advance(self, n_half - 1)
                     self.iter = it + n_half - 1  # colour of the last iteration
-                src = self._fields[self._cur]
                 self._last_half_sweep()
             finally:
                 self.iter = it
+            src = self._fields[1 - self._cur]  # what the last half-sweep read
             st = self._lib.tf_wrap_ghosts_from(_lib.ptr(src), _lib.ptr(self._fields[self._cur]), self.batch_size,
                                                self.Nx, self.Ny, self.Nz, self._stream())
             _lib.check(st, "tf_wrap_ghosts_from")

@@ -45,3 +45,21 @@ def test_periodic_with_other_electrode_values():
         o.run(n)
         s.solve(iter_limit=s.iter + n, verbose=False, conv_crit=0.0)
         assert s._resident and np.array_equal(s.field.cpu().numpy(), o.field.numpy())
+
+
+@pytest.mark.parametrize("cls,ocls", [(tau.Solver, OracleSolver), (tau.PeriodicSolver, OraclePeriodicSolver)])
+@pytest.mark.parametrize("by_hand", [False, True])
+def test_lost_waits_of_solves_that_end_between_checks(cls, ocls, by_hand):
+    """With a single poll per wait the first launch is lost; what it read is
+    not written again before the loss is known."""
+    img = (np.random.default_rng(6).random((40, 44, 46)) < 0.65).astype(np.uint8)
+    s, o = cls(img), ocls(img)
+    assert s._resident_sweep()
+    s._resident.spin = 1
+    for n in (50, 10, 70):
+        o.run(n)
+        s.solve(iter_limit=s.iter + n, verbose=False, conv_crit=0.0)
+        assert s._resident is False, "no wait ran out"
+        if by_hand:
+            s.half_sweeps_per_pass = 4
+    assert np.array_equal(s.field.cpu().numpy(), o.field.numpy())

@@ -4,11 +4,12 @@ whose waits ran out) on a stand-in for the device.
 
 The stand-in's field holds, in every interior voxel, the number of iterations
 behind it, and in its x ghosts the boundary value it was given; a launch
-requires its source to hold the iteration it starts from.  As on the device, a
+requires its source to hold an iteration of its colour.  As on the device, a
 lost resident launch stores its number in the status and leaves dst void, and
 later resident launches write nothing until the status is cleared."""
 import contextlib
 import ctypes
+import random
 
 import numpy as np
 import pytest
@@ -38,8 +39,11 @@ class Device:
     def _run(self, src, dst, n, colour):
         s, d = self._field(src), self._field(dst)
         it = s[1, 1, 1]
-        assert np.all(s[1:-1, 1:-1, 1:-1] == it) and it >= 0, "a void field was read"
-        assert np.all(s[[0, -1]] == self.boundary), "a field with other boundary values was read"
+        assert np.all(s[1:-1, 1:-1, 1:-1] == it)
+        if it == VOID:  # as long as the loss is not known
+            d[1:-1, 1:-1, 1:-1] = VOID
+            return
+        assert np.all(s[[0, -1], 1:-1, 1:-1] == self.boundary), "a field with other boundary values was read"
         assert int(it) & 1 == colour, f"iteration {it} read for a launch of colour {colour}"
         d[1:-1, 1:-1, 1:-1] = it + n
 
@@ -64,7 +68,9 @@ class Device:
             self._run(src, dst, n, colour)
         return 0
 
-    def tf_wrap_ghosts_from(self, *args):
+    def tf_wrap_ghosts_from(self, src, dst, *args):
+        a, b = (self._field(p)[1, 1, 1] for p in (src, dst))
+        assert a == b - 1 or a == b == VOID, "ghosts of another field than the one before"
         return 0
 
     def tf_hbm_copy(self, src, dst, n, stream):
@@ -119,11 +125,14 @@ def make(cls, device, spare=True):
 
     class Stub(cls):
         stop = None  # iteration at which the check finds convergence
+        broken = None  # iteration from which a check is interrupted
 
         def _launch_operands(self, H, tile):
             return self.kind | self._sweep_flags, 0, None, 0, tile
 
         def compute_metrics(self):
+            if self.broken is not None and self.iter >= self.broken:
+                raise KeyboardInterrupt
             flux, _ = self._layer_sums()
             assert self._sums_host[0] == self.iter, "another field was checked"
             done = self.stop is not None and self.iter >= self.stop
@@ -142,7 +151,7 @@ def make(cls, device, spare=True):
     shape = (1, X + 2, Y + 2, Z + 2)
     s._fields = [_lib.slack_buffer(shape, torch.float32, s.device) for _ in range(2)]
     for f in s._fields:
-        f[:, [0, -1]] = device.boundary
+        f[:, [0, -1], 1:-1, 1:-1] = device.boundary
     s._field_init = _lib.slack_buffer(shape, torch.float32, s.device)
     s._copy_field(s._fields[0], s._field_init)
     s._spare = None
@@ -166,7 +175,7 @@ def holds(s, device):
     """The solver's field is that of its iteration, with its boundary."""
     f = s.field[0].numpy()
     assert np.all(f[1:-1, 1:-1, 1:-1] == s.iter), (f[1, 1, 1], s.iter)
-    assert np.all(f[[0, -1]] == device.boundary)
+    assert np.all(f[[0, -1], 1:-1, 1:-1] == device.boundary)
 
 
 def run(s, limit, stop=None):
@@ -192,8 +201,66 @@ def test_boundary_set_before_the_third_buffer(device):
     launch, holds in the third buffer too."""
     s = make(tau.PeriodicSolver, device)
     f = s.field.clone()
-    f[:, [0, -1]] = device.boundary = 0.25
+    f[:, [0, -1], 1:-1, 1:-1] = device.boundary = 0.25
     s.field = f
     run(s, 330)
     assert s._resident.third is not None
+    holds(s, device)
+
+
+@pytest.mark.parametrize("cls", [tau.Solver, tau.PeriodicSolver])
+@pytest.mark.parametrize("lost", [1, 2, 3])
+def test_lost_launch_of_solves_that_end_between_checks(cls, lost, device):
+    """A solve that ends between checks returns a field that is known: a lost
+    launch is repeated before the buffer that it read is written again."""
+    s = make(cls, device)
+    device.lost = {lost}
+    for limit in (50, 60, 130, 250):
+        run(s, limit)
+        assert s.iter == limit and not (s._resident and s._resident.log)
+        holds(s, device)
+    assert s._resident is False
+
+
+@pytest.mark.parametrize("cls", [tau.Solver, tau.PeriodicSolver])
+def test_lost_launch_then_a_hand_set_depth(cls, device):
+    s = make(cls, device)
+    device.lost = {1}
+    run(s, 50)
+    s.half_sweeps_per_pass = 4
+    run(s, 130)
+    holds(s, device)
+
+
+@pytest.mark.parametrize("cls", [tau.Solver, tau.PeriodicSolver])
+@pytest.mark.parametrize("spare", [False, True])
+@pytest.mark.parametrize("seed", range(25))
+def test_any_sequence(cls, spare, seed, device):
+    """Solves to any iteration, converged or not, with the depth set by hand
+    or not, interrupted in a check, resets, new fields, lost launches: the
+    field is always that of the solver's iteration."""
+    rng = random.Random(seed)
+    s = make(cls, device, spare)
+    device.lost = set(rng.sample(range(1, 40), rng.randint(0, 2)))
+    for _ in range(12):
+        act = rng.random()
+        if act < 0.1:
+            s.reset()
+            device.boundary = 0.5
+        elif act < 0.2:
+            f = s.field.clone()
+            f[:, [0, -1], 1:-1, 1:-1] = device.boundary = rng.choice([0.25, 0.5, 1.0])
+            s.field = f
+        elif act < 0.35:
+            s.half_sweeps_per_pass = rng.choice([None, None, 3, 4])
+        elif act < 0.45:
+            s.broken = s.iter + rng.randint(0, 200)
+            with contextlib.suppress(KeyboardInterrupt):
+                run(s, s.iter + 300)
+            s.broken = None
+        else:
+            run(s, s.iter + rng.choice([1, 7, 40, 100, 100 - s.iter % 100, 230]),
+                rng.choice([None, s.iter + 100, s.iter + 200]))
+        if rng.random() < 0.7:
+            holds(s, device)
     holds(s, device)
