@@ -467,7 +467,8 @@ class SORSolver(ABC):
         self._fields, self._cur = [src, other], 0
         self._ahead, self._checked, self._sums_ready = 0, None, None
         end, self.iter = self.iter, it
-        self._advance(end - it)
+        if end > it:  # (else a launch ahead, not taken over yet)
+            self._advance(end - it)
         self.iter = end
 
     def _enqueue_layer_sums(self) -> None:

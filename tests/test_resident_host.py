@@ -264,3 +264,23 @@ def test_any_sequence(cls, spare, seed, device):
         if rng.random() < 0.7:
             holds(s, device)
     holds(s, device)
+
+
+@pytest.mark.parametrize("cls", [tau.Solver, tau.PeriodicSolver])
+def test_field_read_in_a_check_after_a_lost_launch_ahead(cls, device):
+    """The launch ahead of the check at 100 is lost and a check that looks at
+    the field finds out: there is nothing to repeat."""
+    s = make(cls, device)
+    device.lost = {2}
+    metrics = s.compute_metrics
+
+    def look():
+        out = metrics()
+        if s.iter == 100:  # (later checks have streaming launches ahead)
+            holds(s, device)
+        return out
+
+    s.compute_metrics = look
+    run(s, 230)
+    assert s._resident is False
+    holds(s, device)
