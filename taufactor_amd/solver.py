@@ -468,7 +468,9 @@ class SORSolver(ABC):
         self._ahead, self._checked, self._sums_ready = 0, None, None
         end, self.iter = self.iter, it
         if end > it:  # (else a launch ahead, not taken over yet)
-            self._advance(end - it)
+            # (a field may be read with another device current)
+            with torch.cuda.device(self.device):
+                self._advance(end - it)
         self.iter = end
 
     def _enqueue_layer_sums(self) -> None:

@@ -284,3 +284,33 @@ def test_field_read_in_a_check_after_a_lost_launch_ahead(cls, device):
     run(s, 230)
     assert s._resident is False
     holds(s, device)
+
+
+def test_repeated_on_the_solvers_device(device, monkeypatch):
+    """A field read outside of solve() that finds a lost launch repeats it on
+    the solver's device, whichever is current."""
+    current = []
+
+    @contextlib.contextmanager
+    def on(d):
+        current.append(d)
+        try:
+            yield
+        finally:
+            current.pop()
+
+    monkeypatch.setattr(torch.cuda, "device", on)
+    s = make(tau.Solver, device)
+    device.lost = {1}
+    s.broken = 100
+    with contextlib.suppress(KeyboardInterrupt):
+        run(s, 200)
+    sweep = device.tf_sweep
+
+    def checked(*args):
+        assert current and current[-1] == s.device
+        return sweep(*args)
+
+    device.tf_sweep = checked
+    holds(s, device)
+    assert s._resident is False and s.iter == 100
