@@ -578,8 +578,8 @@ class SORSolver(ABC):
                         raise
                     if self.converged:
                         self._drop_ahead()
-            torch.cuda.synchronize(self.device)
             self._settle()
+            torch.cuda.synchronize(self.device)
             self.walltime = timer() - start
             self._end_simulation(self.iter, verbose)
             if self.tau_x is None:

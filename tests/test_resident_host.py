@@ -314,3 +314,16 @@ def test_repeated_on_the_solvers_device(device, monkeypatch):
     device.tf_sweep = checked
     holds(s, device)
     assert s._resident is False and s.iter == 100
+
+
+def test_walltime_includes_a_repetition(device, monkeypatch):
+    """solve() waits for the device after its last launch, that of a
+    repetition too."""
+    s = make(tau.Solver, device)
+    device.lost = {1}
+    calls = []
+    sweep = device.tf_sweep
+    device.tf_sweep = lambda *a: calls.append("sweep") or sweep(*a)
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda d=None: calls.append("wait"))
+    run(s, 50)
+    assert "sweep" in calls and calls[-1] == "wait"
