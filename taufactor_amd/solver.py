@@ -21,6 +21,7 @@ Differences from the reference, all deliberate:
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 
 import math
@@ -555,7 +556,7 @@ class SORSolver(ABC):
         if verbose == "debug":
             self.tau_t = []
 
-        with torch.no_grad(), torch.cuda.device(self.device):
+        with torch.no_grad(), torch.cuda.device(self.device), _turns(self.device):
             start = timer()
             # apply_boundary_conditions before every iteration (reference
             # loop) is part of _advance: the ghosts of the open solvers are
@@ -633,11 +634,31 @@ class SORSolver(ABC):
                   f"{torch.cuda.max_memory_reserved(device=self.device) / 1e6:.2f} MB reserved)")
 
 
-# the stream of the latest resident launch of each device: two of them at once
-# would wait for each other's compute units until their waits run out, so one
-# on another stream is ordered after it
+# (stream, thread) of the latest resident launch of each device by a solve
+# that is still running, or (event after it, None) of one that was interrupted:
+# two of them at once would wait for each other's compute units until their
+# waits run out, so one on another stream is ordered after it.  A solve that
+# ends takes its stream out, which its owner may destroy from then on (an event
+# after every launch instead took 3 % of a 256^3 periodic solve)
 _resident_turn: dict = {}
 _resident_lock = threading.Lock()
+
+
+@contextlib.contextmanager
+def _turns(device):
+    """Around a solve, which leaves its device idle unless it is interrupted."""
+    idle = False
+    try:
+        yield
+        idle = True
+    finally:
+        with _resident_lock:
+            last, thread = _resident_turn.get(device.index) or (None, None)
+            if thread == threading.get_ident():
+                if idle:
+                    del _resident_turn[device.index]
+                else:
+                    _resident_turn[device.index] = last.record_event(), None
 
 
 class _ResidentSweep:
@@ -690,8 +711,10 @@ class _ResidentSweep:
         volume = 4 * (X + 2) * (Y + 2) * (Z + 2)  # bytes of a field (and of face words)
         table = _lib.ptr(self.table) if self.table is not None else None
         with _resident_lock:
-            last = _resident_turn.get(s.device.index)
-            if last is not None and last != stream:
+            last, thread = _resident_turn.get(s.device.index) or (stream, None)
+            if thread is None and last is not stream:
+                stream.wait_event(last)
+            elif last != stream:
                 stream.wait_event(last.record_event())
             for b in range(0, B, self.per):
                 if self.tag + n + 1 >= 2 ** 32:
@@ -705,7 +728,7 @@ class _ResidentSweep:
                 if st != 0:
                     break
                 self.tag += n + 1
-            _resident_turn[s.device.index] = stream
+            _resident_turn[s.device.index] = stream, threading.get_ident()
         if st == _lib.NOT_RESIDENT and not self.log:
             s._resident = False
             return False

@@ -10,6 +10,7 @@ later resident launches write nothing until the status is cleared."""
 import contextlib
 import ctypes
 import random
+import threading
 
 import numpy as np
 import pytest
@@ -327,3 +328,81 @@ def test_walltime_includes_a_repetition(device, monkeypatch):
     monkeypatch.setattr(torch.cuda, "synchronize", lambda d=None: calls.append("wait"))
     run(s, 50)
     assert "sweep" in calls and calls[-1] == "wait"
+
+
+class _Turn:
+    """Streams and events that note what was asked of them."""
+
+    def __init__(self, monkeypatch, device):
+        self.log = []
+        self.stream_of = {}  # of each thread
+        turn = self
+
+        class Event(_Event):
+            def record(self, stream=None):
+                self.at = device.launches
+
+        class Stream:
+            def __init__(self, handle):
+                self.cuda_stream, self.gone = handle, False
+
+            def __eq__(self, other):
+                return self.cuda_stream == other.cuda_stream
+
+            def wait_event(self, e):
+                turn.log.append((self.cuda_stream, e.at))
+
+            def record_event(self, e=None):
+                assert not self.gone, "a stream that is gone was used"
+                e = e or Event()
+                e.record(self)
+                return e
+
+        self.stream = Stream
+        monkeypatch.setattr(torch.cuda, "Event", Event)
+        monkeypatch.setattr(torch.cuda, "current_stream", lambda d=None: self.stream_of[threading.get_ident()])
+
+    def run(self, stream, s, limit):
+        self.stream_of[threading.get_ident()] = stream
+        run(s, limit)
+
+
+@pytest.mark.parametrize("interrupted", [False, True])
+def test_a_stream_that_is_gone(interrupted, device, monkeypatch):
+    """A solve on a stream that is destroyed after it, then one on another
+    stream: the first stream is not used again, and launches that an
+    interrupted solve left on it are waited for."""
+    turn = _Turn(monkeypatch, device)
+    first, second = make(tau.Solver, device), make(tau.Solver, device)
+    a, b = turn.stream(1), turn.stream(2)
+    first.broken = 100 if interrupted else None
+    with contextlib.suppress(KeyboardInterrupt):
+        turn.run(a, first, 150)
+    launches = device.launches
+    a.gone = True
+    turn.run(b, second, 50)
+    assert turn.log == ([(2, launches)] if interrupted else [])
+
+
+def test_turns_of_threads(device, monkeypatch):
+    """A solve on a stream of its own in another thread, while the first one
+    stands in a check: each waits for the other's launches."""
+    turn = _Turn(monkeypatch, device)
+    first, second = make(tau.Solver, device), make(tau.Solver, device)
+    a, b = turn.stream(1), turn.stream(2)
+    metrics = first.compute_metrics
+
+    def meanwhile():
+        if first.iter == 100:
+            t = threading.Thread(target=turn.run, args=(b, second, 50))
+            t.start()
+            t.join()
+        return metrics()
+
+    first.compute_metrics = meanwhile
+    turn.run(a, first, 150)
+    # launches 1, 2 (ahead) and 4 of the first solve, 3 of the second, which
+    # had ended before 4
+    assert turn.log == [(2, 2)]
+    assert first.iter == 150 and second.iter == 50
+    assert solver_module._resident_turn == {}
