@@ -333,8 +333,11 @@ class SORSolver(ABC):
         first self._ahead of them were launched ahead of the last check.
         resident False: with streaming launches in any case."""
         resident = resident and self._resident_sweep()
-        if not resident and self._resident and any(src is f for _, src, _ in self._resident.log for f in self._fields):
-            self._settle()  # a field that a lost launch would be repeated from must not be written
+        if not resident and self._resident:
+            # a field that a lost launch would be repeated from must not be written
+            written = self._fields if n_half > 1 else [self._fields[1 - self._cur]]
+            if any(src is f for _, src, _ in self._resident.log for f in written):
+                self._settle()
         done, self._ahead = self._ahead, 0
         it = self.iter + done
         n_half -= done
