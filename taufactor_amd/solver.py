@@ -90,7 +90,7 @@ class SORSolver(ABC):
         self._launch_events = None
         self._codes = None
         self._sweep_codes = None
-        self._groups = None  # see Solver._sweep_groups
+        self._groups = None  # see Solver._sweep_groups (False: no memory for them)
         self._hm_lut = None
         self._n_classes = 0
         self._spans_cache = {}
@@ -687,7 +687,10 @@ class _ResidentSweep:
             if r < 0:
                 _lib.check(r, "tf_resident_plan")
             if r:
-                return cls(s, kind, per, plan)
+                try:
+                    return cls(s, kind, per, plan)
+                except torch.cuda.OutOfMemoryError:
+                    return None  # the streaming sweep needs no more memory than the fields
         return None
 
     def __init__(self, s, kind, per, plan):
@@ -696,6 +699,10 @@ class _ResidentSweep:
         self.mail = torch.zeros(plan.mail_bytes // 8, dtype=torch.int64, device=s.device)
         self.status = s._sums[-1:].view(torch.int32)[:1]
         self.third = None  # see _PeriodicYZ._last_half_sweep
+        if s._sweep_flags:
+            self.third = _lib.slack_buffer(tuple(s._field_init.shape), torch.float32, s.device)
+            # (the x ghosts may have been set since the set-up)
+            s._copy_field(s._fields[s._cur], self.third)
         self.spin = 0
         self.tag, self.count = 1, 0
         self.log = []  # (number, field read, first iteration) of each launch
@@ -996,10 +1003,16 @@ class Solver(ThroughTransportSolver):
         voxels = self.batch_size * self.Nx * self.Ny * self.Nz
         if self.kind != _lib.KIND_SOLVER or self._sweep_flags or voxels < autotune.MIN_VOXELS:
             return None
+        if self._groups is False:
+            return None
         if self._groups is None:
             B, X, Y, Z = self.batch_size, self.Nx, self.Ny, self.Nz
             n = B * int(self._lib.tf_sweep_groups_bytes(X, Y, Z))
-            self._groups = torch.empty(n, dtype=torch.uint8, device=self.device)
+            try:
+                self._groups = torch.empty(n, dtype=torch.uint8, device=self.device)
+            except torch.cuda.OutOfMemoryError:
+                self._groups = False  # the volume sweeps without them
+                return None
             st = self._lib.tf_pack_sweep_groups(_lib.ptr(self._codes), _lib.ptr(self._groups), B, X, Y, Z,
                                                 self._stream())
             _lib.check(st, "tf_pack_sweep_groups")
@@ -1523,10 +1536,6 @@ class _PeriodicYZ:
         is kept until the launch is known to have run to its end."""
         r = self._resident
         if r and r.log:
-            if r.third is None:
-                r.third = _lib.slack_buffer(tuple(self._field_init.shape), torch.float32, self.device)
-                # (the x ghosts may have been set since the set-up)
-                self._copy_field(self._fields[self._cur], r.third)
             k = 1 - self._cur
             self._fields[k], r.third = r.third, self._fields[k]
         SORSolver._advance(self, 1, resident=False)

@@ -421,3 +421,32 @@ def test_no_wait_for_the_status_inside_a_solve(cls, device):
     s._settle = lambda: asked.append(s.iter) or settle()
     run(s, 1000, stop=500)
     assert asked == [500]
+
+
+@pytest.mark.parametrize("cls", [tau.Solver, tau.PeriodicSolver])
+@pytest.mark.parametrize("what", ["zeros", "slack_buffer"])
+def test_no_memory_for_the_resident_sweep(cls, what, device, monkeypatch):
+    """A solver whose mailbox or third buffer does not fit streams."""
+    s = make(cls, device)
+
+    def full(*args, **kwargs):
+        raise torch.cuda.OutOfMemoryError("full")
+
+    monkeypatch.setattr(torch if what == "zeros" else _lib, what, full)
+    run(s, 230)
+    assert bool(s._resident) == (what == "slack_buffer" and cls is tau.Solver)
+    holds(s, device)
+
+
+def test_no_memory_for_code_groups(device, monkeypatch):
+    """A volume whose codes in groups do not fit sweeps without them."""
+    s = make(tau.Solver, device)
+    device.tf_sweep_groups_bytes = lambda *a: 64
+
+    def full(*args, **kwargs):
+        raise torch.cuda.OutOfMemoryError("full")
+
+    monkeypatch.setattr(solver_module.autotune, "MIN_VOXELS", 0)
+    monkeypatch.setattr(torch, "empty", full)
+    assert s._sweep_groups() is None
+    assert s._sweep_groups() is None and not device.launches
