@@ -233,9 +233,10 @@ class SORSolver(ABC):
     def _launch_config(self):
         """(H, tile) of the next launches: explicit settings win; otherwise the
         autotuner's choice for volumes of at least autotune.MIN_VOXELS voxels
-        (made once, before the first iteration), for smaller ones with
-        neither set autotune.small_volume_default, else H = 4 and the
-        library's default tile."""
+        (made once, before the first iteration or where the solver leaves the
+        resident sweep), for smaller ones with neither set
+        autotune.small_volume_default, else H = 4 and the library's default
+        tile."""
         H, tile = self.half_sweeps_per_pass, self.tile
         if H is not None and tile is not None:
             return int(H), tuple(tile)
@@ -244,12 +245,14 @@ class SORSolver(ABC):
         if H is None and tile is None and self.autotune and self._tunable and not big:
             sH, stile = autotune.small_volume_default(voxels)
             return (sH or DEFAULT_HALF_SWEEPS_PER_PASS), stile
-        if self._auto_cfg is None:
-            if self.autotune and self._tunable and big and self.iter == 0:
-                self._auto_cfg = autotune.tune_solver(self, H, tile)
-            else:
-                self._auto_cfg = (None, None)
-        aH, atile = self._auto_cfg
+        auto = self._auto_cfg
+        if auto is None:
+            auto = (None, None)
+            if self.autotune and self._tunable and big and (self.iter == 0 or self._resident is False):
+                auto = autotune.tune_solver(self, H, tile)
+            if not self._resident:  # (else a periodic solver's half-sweep between resident launches)
+                self._auto_cfg = auto
+        aH, atile = auto
         H = int(H) if H is not None else (aH or DEFAULT_HALF_SWEEPS_PER_PASS)
         tile = tuple(tile) if tile is not None else atile
         return H, tile

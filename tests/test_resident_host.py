@@ -450,3 +450,19 @@ def test_no_memory_for_code_groups(device, monkeypatch):
     monkeypatch.setattr(torch, "empty", full)
     assert s._sweep_groups() is None
     assert s._sweep_groups() is None and not device.launches
+
+
+@pytest.mark.parametrize("cls", [tau.Solver, tau.PeriodicSolver])
+def test_tuned_after_a_lost_launch(cls, device, monkeypatch):
+    """A large volume that leaves the resident sweep is tuned as one that
+    streams from the start, and not before."""
+    tuned = []
+    monkeypatch.setattr(solver_module.autotune, "MIN_VOXELS", 1)
+    monkeypatch.setattr(solver_module.autotune, "tune_solver", lambda s, H, tile: tuned.append(s.iter) or (3, (8, 2, 0)))
+    s = make(cls, device)
+    device.lost = {4}
+    run(s, 150)
+    assert not tuned and s._resident
+    run(s, 400)
+    assert len(tuned) == 1 and s._resident is False and s._launch_config() == (3, (8, 2, 0))
+    holds(s, device)
