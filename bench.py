@@ -102,7 +102,7 @@ def sweep_kernel(s, kind: str, H: int, tile):
     """(half-sweeps per timed launch, kernel, its compilation unit) of the
     sweep that solver s ran: a resident launch counts its half-sweeps, and
     large Solver volumes read their codes in groups."""
-    if s._resident:
+    if s._resident_wanted():
         return 1, f"k_resident<{kind}>", None
     if s._groups is not None and s._launch_operands(H, _tile(tile))[0] != s.kind:
         return H, f"k_sweep<{H}, {kind}Groups, {tile[0]}, {tile[1]}>", "sweep_solver_groups.hip"

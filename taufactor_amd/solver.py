@@ -248,9 +248,10 @@ class SORSolver(ABC):
         auto = self._auto_cfg
         if auto is None:
             auto = (None, None)
-            if self.autotune and self._tunable and big and (self.iter == 0 or self._resident is False):
+            left = self._resident is not None and not self._resident_wanted()
+            if self.autotune and self._tunable and big and (self.iter == 0 or left):
                 auto = autotune.tune_solver(self, H, tile)
-            if not self._resident:  # (else a periodic solver's half-sweep between resident launches)
+            if not self._resident_wanted():  # (else a periodic solver's half-sweep between resident launches)
                 self._auto_cfg = auto
         aH, atile = auto
         H = int(H) if H is not None else (aH or DEFAULT_HALF_SWEEPS_PER_PASS)
@@ -335,6 +336,7 @@ class SORSolver(ABC):
         """Run n_half reference iterations (half-sweeps) on the device; the
         first self._ahead of them were launched ahead of the last check.
         resident False: with streaming launches in any case."""
+        timed = resident and self._resident_chosen() and self._resident.measured
         resident = resident and self._resident_sweep()
         if not resident and self._resident:
             # a field that a lost launch would be repeated from must not be written
@@ -344,8 +346,13 @@ class SORSolver(ABC):
         done, self._ahead = self._ahead, 0
         it = self.iter + done
         n_half -= done
-        if n_half > 0 and resident and self._resident.launch(self, n_half, it):
-            return
+        with self._resident.time(n_half) if timed and self._resident else contextlib.nullcontext():
+            if n_half > 0 and resident and self._resident.launch(self, n_half, it):
+                return
+            self._stream_launches(n_half, it)
+
+    def _stream_launches(self, n_half: int, it: int) -> None:
+        """n_half half-sweeps from iteration it as streaming launches."""
         per, tile = self._sweep_args()
         # timing (bench.py): HIP events on the launch stream around the
         # launches that fuse the full `per` half-sweeps (a shorter last
@@ -394,6 +401,8 @@ class SORSolver(ABC):
             if self._resident.launch(self, n, self.iter):
                 self._ahead = n
                 return
+        if self._resident and self._resident.log:
+            return  # the first of them would write what the block's launch, not known to have run, read
         per, tile = self._sweep_args()
         launches = 1
         if self._spare is not None:
@@ -428,15 +437,22 @@ class SORSolver(ABC):
     # iterations launched ahead of a check decision by the resident sweep
     RESIDENT_AHEAD = 40
 
-    def _resident_sweep(self) -> bool:
-        """Do the launches of this solver run as resident sweeps?  Where the
-        kind has one and the volume fits the device (tf_resident_plan),
-        unless the launch configuration was set by hand."""
+    def _resident_chosen(self) -> bool:
+        """Does this solver have a resident sweep?  Where the kind has one and
+        the volume fits the device (tf_resident_plan), unless the launch
+        configuration was set by hand."""
         if self.half_sweeps_per_pass is not None or self.tile is not None:
             return False
         if self._resident is None:
             self._resident = _ResidentSweep.make(self) or False
         return bool(self._resident)
+
+    def _resident_wanted(self) -> bool:
+        return bool(self._resident) and self._resident.wanted()
+
+    def _resident_sweep(self) -> bool:
+        """Do the next launches of this solver run as resident sweeps?"""
+        return self._resident_chosen() and self._resident_wanted()
 
     def _resident_kind(self):
         """Kind (with the sweep flags) of this solver's resident sweep, None
@@ -667,6 +683,36 @@ def _turns(device):
                     _resident_turn[device.index] = last.record_event(), None
 
 
+# (device, kinds, layout and shape of a solver) -> is its resident sweep the
+# faster one?  Measured, see _ResidentSweep.time
+_resident_faster: dict = {}
+
+
+def _resident_unsure(kind, p, per: int, B: int, X: int, Y: int, Z: int, cus: int) -> bool:
+    """Layouts whose half-sweeps are not always shorter than the streaming
+    sweep's.  Whole solves of 400 iterations, streaming over resident, on
+    MI355X:
+    * several launches per half-sweep for a batch: 2.3 (MultiPhase, 256 x
+      16^3) to 0.35 (256 x 40^3, 10 launches) with no simple order; with at
+      least three quarters of the lanes' elements filled, the per-voxel field
+      1.3 to 1.8;
+    * rows of more than 512 voxels (16 or 32 per lane: every face message is
+      that much longer): 0.37 (2 x 16 x 1500) to 1.6 (1000 x 4 x 520); rows
+      of pixels of an image only with 32 per lane and fewer than 16 rows
+      (0.81 to 0.96; 1.1 and more with 20);
+    * rows of more than 256 voxels, one to three layers: 0.76 to 1.03; with
+      four 1.0 to 1.8;
+    * rows of at most 56 voxels, two of which share a wave of the streaming
+      sweep, in the largest patches: 0.89 to 1.08.
+    All others measured, 2500 volumes of every kind, gain or are level."""
+    if p.lane_y:
+        return p.elems == 32 and X < 16
+    fill = per * X * Y * Z / (cus * p.waves * 64 * p.px * p.py * p.elems)
+    if per < B and not (kind == _lib.KIND_FIELD and fill >= 0.75):
+        return True
+    return p.elems >= 16 or p.elems == 8 and X < 4 or p.elems * p.px * p.py > 64 and Z <= 56
+
+
 class _ResidentSweep:
     """The resident sweep of one solver (tf_sweep_resident): its layout,
     mailbox and the launches not yet known to have run to their end."""
@@ -691,12 +737,12 @@ class _ResidentSweep:
                 _lib.check(r, "tf_resident_plan")
             if r:
                 try:
-                    return cls(s, kind, per, plan)
+                    return cls(s, kind, per, plan, cus)
                 except torch.cuda.OutOfMemoryError:
                     return None  # the streaming sweep needs no more memory than the fields
         return None
 
-    def __init__(self, s, kind, per, plan):
+    def __init__(self, s, kind, per, plan, cus):
         self.kind, self.per, self.plan = kind, per, plan
         self.codes, self.table, self.n_table = s._resident_operands()
         self.mail = torch.zeros(plan.mail_bytes // 8, dtype=torch.int64, device=s.device)
@@ -709,6 +755,35 @@ class _ResidentSweep:
         self.spin = 0
         self.tag, self.count = 1, 0
         self.log = []  # (number, field read, first iteration) of each launch
+        shape = (s.batch_size, s.Nx, s.Ny, s.Nz)
+        self.measured = _resident_unsure(kind, plan, per, *shape, cus)
+        self.key = (s.device.index, kind, s.kind, per, *shape)
+        self.times = []  # (start, end, half-sweeps) of check periods
+
+    def wanted(self) -> bool:
+        """Should the next launches be resident?  Unsure layouts find out
+        over the first four long stretches of iterations, two resident, then
+        two streaming, the second of each timed; the next solver of the shape
+        knows."""
+        if not self.measured:
+            return True
+        faster = _resident_faster.get(self.key)
+        if faster is None and len(self.times) == 4 and self.times[3][1].query():
+            res, stream = (t0.elapsed_time(t1) / n for t0, t1, n in self.times[1::2])
+            faster = _resident_faster[self.key] = res <= stream
+        return len(self.times) < 2 if faster is None else faster
+
+    @contextlib.contextmanager
+    def time(self, n: int):
+        """Around the launches of n half-sweeps of an unsure layout."""
+        if n < CHECK_EVERY // 2 or len(self.times) == 4 or self.key in _resident_faster:
+            yield
+            return
+        t0, t1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        t0.record()
+        yield
+        t1.record()
+        self.times.append((t0, t1, n))
 
     def launch(self, s, n: int, it: int) -> bool:
         """n half-sweeps from iteration it; False if the device does not hold

@@ -5,6 +5,7 @@ import pytest
 
 import taufactor_amd as tau
 from oracle.restate import OracleMultiPhaseSolver, OraclePeriodicSolver, OracleSolver
+from taufactor_amd import solver
 
 pytestmark = pytest.mark.gpu
 
@@ -63,3 +64,19 @@ def test_lost_waits_of_solves_that_end_between_checks(cls, ocls, by_hand):
         if by_hand:
             s.half_sweeps_per_pass = 4
     assert np.array_equal(s.field.cpu().numpy(), o.field.numpy())
+
+
+@pytest.mark.parametrize("cls,ocls,shape", [(tau.Solver, OracleSolver, (5, 9, 600)), (tau.Solver, OracleSolver, (14, 1030)),
+                                            (tau.PeriodicSolver, OraclePeriodicSolver, (6, 8, 1024)),
+                                            (tau.MultiPhaseSolver, OracleMultiPhaseSolver, (3, 7, 300))])
+def test_measured_against_the_streaming_sweep(cls, ocls, shape):
+    """Layouts of which it is not known which sweep is the faster change from
+    one to the other inside a solve; the next solver takes the faster one."""
+    extra = (dict(D3),) if cls is tau.MultiPhaseSolver else ()
+    img = _labels(shape, 3 if extra else 2, 9) if extra else (np.random.default_rng(9).random(shape) < 0.8).astype(np.uint8)
+    field = ocls(img, *extra).run(630).field.numpy()
+    for _ in range(2):
+        s = cls(img, *extra)
+        s.solve(iter_limit=630, verbose=False, conv_crit=0.0)
+        assert s._resident.measured and s._resident.key in solver._resident_faster
+        assert np.array_equal(s.field.cpu().numpy(), field)

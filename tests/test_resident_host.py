@@ -30,6 +30,8 @@ class Device:
         self.lost = set()  # resident launches (counted from 1) whose waits run out
         self.launches = 0
         self.boundary = 0.5
+        self.clock, self.cost = 0.0, {"resident": 1.0, "streaming": 2.0}  # time of a half-sweep
+        self.ran = []  # (path, half-sweeps) of each launch
         self.status = None  # of the solver made last
         self.solver = None
 
@@ -47,7 +49,12 @@ class Device:
         assert int(it) & 1 == colour, f"iteration {it} read for a launch of colour {colour}"
         d[1:-1, 1:-1, 1:-1] = it + n
 
+    def took(self, path, n):
+        self.clock += self.cost[path] * n
+        self.ran.append((path, n))
+
     def tf_sweep(self, src, dst, codes, hm, n_table, kind, B, nx, ny, nz, w, colour, h, tile, stream):
+        self.took("streaming", h)
         r = self.solver._resident
         if r and self.status is not None and self.status[0] and any(e[0] >= self.status[0] for e in r.log):
             # the host does not know of the loss yet: whatever was read
@@ -57,13 +64,15 @@ class Device:
         return 0
 
     def tf_resident_plan(self, kind, B, nx, ny, nz, cus, plan):
-        plan._obj.mail_bytes = 64
+        p = plan._obj
+        p.elems, p.px, p.py, p.waves, p.wy, p.tiles, p.mail_bytes = 2, 1, 1, 16, 4, 1, 64
         return 1
 
     def tf_sweep_resident(self, src, dst, codes, table, n_table, kind, B, nx, ny, nz, w, colour, n, plan, section,
                           mail, mail_bytes, tag, status, launch_id, spin, stream):
         st = self.status = self._view(status, ctypes.c_int32, 1)
         self.launches += 1
+        self.took("resident", n)
         if st[0]:
             return 0
         if self.launches in self.lost:
@@ -89,14 +98,22 @@ class Device:
 
 
 class _Event:
+    device = None
+
     def __init__(self, *a, **k):
         pass
 
     def record(self, *a):
-        pass
+        self.at = self.device.clock
 
     def synchronize(self):
         pass
+
+    def query(self):
+        return True
+
+    def elapsed_time(self, end):
+        return end.at - self.at
 
 
 class _Stream:
@@ -122,7 +139,9 @@ def device(monkeypatch):
         monkeypatch.setattr(torch.cuda, name, f)
     monkeypatch.setattr(solver_module, "_resident_turn", {})
     monkeypatch.setattr(_lib, "stream_handle", lambda d: _Stream.cuda_stream)
-    return Device()
+    monkeypatch.setattr(solver_module, "_resident_faster", {})
+    _Event.device = Device()
+    return _Event.device
 
 
 def make(cls, device, spare=True):
@@ -239,12 +258,17 @@ def test_lost_launch_then_a_hand_set_depth(cls, device):
 
 @pytest.mark.parametrize("cls", [tau.Solver, tau.PeriodicSolver])
 @pytest.mark.parametrize("spare", [False, True])
+@pytest.mark.parametrize("measured", [None, "resident", "streaming"])
 @pytest.mark.parametrize("seed", range(25))
-def test_any_sequence(cls, spare, seed, device):
+def test_any_sequence(cls, spare, measured, seed, device, monkeypatch):
     """Solves to any iteration, converged or not, with the depth set by hand
-    or not, interrupted in a check, resets, new fields, lost launches: the
-    field is always that of the solver's iteration."""
+    or not, interrupted in a check, resets, new fields, lost launches, the two
+    sweeps measured against each other: the field is always that of the
+    solver's iteration."""
     rng = random.Random(seed)
+    if measured:
+        monkeypatch.setattr(solver_module, "_resident_unsure", lambda *a: True)
+        device.cost[measured] = 0.5
     s = make(cls, device, spare)
     device.lost = set(rng.sample(range(1, 40), rng.randint(0, 2)))
     for _ in range(12):
@@ -466,3 +490,53 @@ def test_tuned_after_a_lost_launch(cls, device, monkeypatch):
     run(s, 400)
     assert len(tuned) == 1 and s._resident is False and s._launch_config() == (3, (8, 2, 0))
     holds(s, device)
+
+
+@pytest.mark.parametrize("cls", [tau.Solver, tau.PeriodicSolver])
+@pytest.mark.parametrize("faster", ["resident", "streaming"])
+def test_unsure_layouts_are_measured(cls, faster, device, monkeypatch):
+    """Two periods resident, two streaming, then the faster of them; the next
+    solver of the shape starts with that one, one of another shape does not."""
+    monkeypatch.setattr(solver_module, "_resident_unsure", lambda *a: True)
+    device.cost[faster] = 0.5
+
+    def main(s, n):
+        """The path of each period's launches (a periodic one ends on a
+        streaming half-sweep), without those ahead of a check."""
+        out = []
+        for _ in range(n):
+            del device.ran[:]
+            run(s, s.iter + 100)
+            out.append(max(device.ran, key=lambda r: r[1])[0])
+        holds(s, device)
+        return out
+
+    assert main(make(cls, device), 7) == ["resident"] * 2 + ["streaming"] * 2 + [faster] * 3
+    assert main(make(cls, device), 2) == [faster] * 2
+    s = make(cls, device)
+    s.solve(iter_limit=1000, verbose=False)
+    holds(s, device)
+    monkeypatch.setattr(solver_module, "_resident_faster", {})
+    s = make(cls, device)
+    s.solve(iter_limit=1000, verbose=False)
+    holds(s, device)
+    assert list(solver_module._resident_faster.values()) == [faster == "resident"]
+
+
+def test_which_layouts_are_unsure():
+    """On both sides of each line: ordinary volumes and images are not."""
+    def unsure(kind, shape, per=None):
+        B, X, Y, Z = shape
+        p = _lib.Resident()
+        assert _lib.load().tf_resident_plan(kind, per or B, X, Y, Z, 256, ctypes.byref(p)) == 1
+        return solver_module._resident_unsure(kind, p, per or B, B, X, Y, Z, 256)
+
+    S, F, M = _lib.KIND_SOLVER, _lib.KIND_FIELD, _lib.KIND_MULTIPHASE_FACES
+    for kind, shape in [(S, (1, 32, 32, 32)), (S, (1, 203, 157, 181)), (S, (1, 256, 256, 256)), (S, (4, 96, 96, 96)),
+                        (S, (1, 611, 803, 1)), (S, (1, 16, 1030, 1)), (S, (1, 4, 300, 300)), (S, (1, 2, 300, 256)),
+                        (S, (1, 40, 40, 512)), (S, (1, 350, 350, 60)), (F, (1, 128, 128, 128)), (M, (1, 160, 160, 160))]:
+        assert not unsure(kind, shape)
+    assert not unsure(F, (4, 128, 128, 128), 2) and unsure(F, (4, 100, 100, 100), 2)
+    assert unsure(M, (4, 128, 128, 128), 2)
+    for shape in [(1, 15, 1030, 1), (1, 3, 300, 300), (1, 40, 40, 513), (1, 8, 8, 2000), (1, 350, 350, 56)]:
+        assert unsure(S, shape)
