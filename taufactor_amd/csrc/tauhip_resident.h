@@ -657,32 +657,33 @@ __global__ __launch_bounds__(NW * 64) void k_resident(ResidentArgs a) {
             step(ic<Q0 ^ 1>{}, t + 1);
         }
     } else {
-    for (int t = 0; t < a.n_half; ++t) {
-        const bool odd = ((q0 ^ t) & 1) != 0;
-        if constexpr (NBUF == 2) {
-            if (live) {
-                if (odd) {
-                    half(ic<1>{}, t);
-                    publish(ic<1>{}, t & 1);
-                } else {
-                    half(ic<0>{}, t);
-                    publish(ic<0>{}, t & 1);
+        // the patches differ in their first colour: a branch per wave, the
+        // barriers outside of it
+        for (int t = 0; t < a.n_half; ++t) {
+            const bool odd = ((q0 ^ t) & 1) != 0;
+            if constexpr (NBUF == 2) {
+                if (live) {
+                    if (odd) {
+                        half(ic<1>{}, t);
+                        publish(ic<1>{}, t & 1);
+                    } else {
+                        half(ic<0>{}, t);
+                        publish(ic<0>{}, t & 1);
+                    }
+                }
+            } else {
+                if (live) {
+                    if (odd) half(ic<1>{}, t);
+                    else half(ic<0>{}, t);
+                }
+                __syncthreads();  // the edges have been read
+                if (live) {
+                    if (odd) publish(ic<1>{}, 0);
+                    else publish(ic<0>{}, 0);
                 }
             }
-        } else {
-            if (live) {
-                if (odd) half(ic<1>{}, t);
-                else half(ic<0>{}, t);
-            }
-            __syncthreads();  // the edges have been read
-            if (live) {
-                if (odd) publish(ic<1>{}, 0);
-                else publish(ic<0>{}, 0);
-            }
+            __syncthreads();
         }
-        __syncthreads();
-    }
-
     }
 
     if (!live) return;
@@ -737,9 +738,11 @@ static int launch_resident(const ResidentArgs& a, hipStream_t st) {
 // The compiled shapes, those that some volume's plan takes: (voxels per lane
 // and row, patch rows in x, patch rows of the other axis, waves).  Up to 32
 // voxels per lane the workgroup has 16 waves (128 registers per lane); larger
-// patches need 8 (256 registers).  No loop spills more than a few registers:
-// a reload waits for every store before it, so one between the sends waits a
-// microsecond for their acknowledgement.  That bounds each kind's patches.
+// patches need 8 (256 registers).  A spilled register's reload waits for
+// every store before it, so one between the sends waits a microsecond for
+// their acknowledgement.  That bounds each kind's patches; four kernels spill
+// (face codes 8, 2, 4 15 registers in either colour and 8, 2, 3 2, field
+// 4, 3, 3 8).
 #define TF_RESIDENT_SHAPES_PAIRS(F) \
     F(2, 1, 1, 16) F(2, 1, 2, 16) F(2, 2, 2, 16) F(2, 2, 4, 16) F(2, 4, 4, 16) F(2, 6, 8, 8) \
     F(4, 1, 1, 16) F(4, 1, 2, 16) F(4, 2, 2, 16) F(4, 2, 3, 16) F(4, 2, 4, 16) F(4, 4, 6, 8) \

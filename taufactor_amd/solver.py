@@ -434,7 +434,13 @@ class SORSolver(ABC):
             self._ahead = 0
         self._checked = None
 
-    # iterations launched ahead of a check decision by the resident sweep
+    # iterations launched ahead of a check decision by the resident sweep: fewer
+    # end before the decision (about 60 us), more are waited for when the solve
+    # converges and drops them.  ms per solve on MI355X with 1, 20, 40, 60, 99:
+    # 32^3 0.73 0.70 0.68 0.69 0.75, 100^3 1.41 1.27 1.19 1.22 1.28, 128^3 electrode
+    # 2.38 2.13 1.89 1.84 1.91, seven phases 121 x 130 x 143 2.27 2.19 2.27 2.37
+    # 2.55, 203 x 157 x 181 5.17 4.95 5.05 5.13 5.29, periodic 256^3 7.39 7.33 7.44
+    # 7.57 7.53
     RESIDENT_AHEAD = 40
 
     def _resident_chosen(self) -> bool:
@@ -726,8 +732,10 @@ class _ResidentSweep:
         cus = torch.cuda.get_device_properties(s.device).multi_processor_count
         # the kinds with face conductances also run batches in several
         # launches (groups of equally many volumes): 0.7 ps per voxel and
-        # half-sweep of 4 x 128^3 against 1.6 streaming; the others stream a
-        # batch that does not fit at once, at 0.5 to 0.7 ps
+        # half-sweep of 4 x 128^3 against 1.6 streaming (other sizes: see
+        # _resident_unsure).  The others stream a batch that does not fit at
+        # once: the Solver kind at 0.5 to 0.7 ps; for the anisotropic and
+        # electrode kinds groups were not measured
         B = s.batch_size
         most = B if kind in (_lib.KIND_FIELD, _lib.KIND_MULTIPHASE_FACES) else 1
         for groups in range(1, most + 1):
@@ -796,7 +804,9 @@ class _ResidentSweep:
             t0, t1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
             t0.record()
         stream = torch.cuda.current_stream(s.device)
-        volume = 4 * (X + 2) * (Y + 2) * (Z + 2)  # bytes of a field (and of face words)
+        # bytes of a field, and of the codes of the kinds that run in groups (a
+        # word per padded voxel; the other kinds have one group, b = 0)
+        volume = 4 * (X + 2) * (Y + 2) * (Z + 2)
         table = _lib.ptr(self.table) if self.table is not None else None
         with _resident_lock:
             last, thread = _resident_turn.get(s.device.index) or (stream, None)
