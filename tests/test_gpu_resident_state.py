@@ -4,7 +4,8 @@ import numpy as np
 import pytest
 
 import taufactor_amd as tau
-from oracle.restate import OracleMultiPhaseSolver, OraclePeriodicSolver, OracleSolver
+from oracle.restate import (OracleAnisotropicSolver, OracleElectrodeSolver, OracleFieldSolver, OracleMultiPhaseSolver,
+                            OraclePeriodicElectrodeSolver, OraclePeriodicSolver, OracleSolver)
 from taufactor_amd import solver
 
 pytestmark = pytest.mark.gpu
@@ -80,3 +81,29 @@ def test_measured_against_the_streaming_sweep(cls, ocls, shape):
         s.solve(iter_limit=630, verbose=False, conv_crit=0.0)
         assert s._resident.measured and s._resident.key in solver._resident_faster
         assert np.array_equal(s.field.cpu().numpy(), field)
+
+
+@pytest.mark.parametrize("kind", ["field", "multiphase", "anisotropic", "electrode", "periodic electrode"])
+def test_lost_waits_of_every_kind(kind):
+    """With a single poll per wait a launch is lost, the solver knows, and its
+    field is the repeated one."""
+    shape = (40, 44, 46)
+    if kind == "field":
+        k = np.random.default_rng(4).uniform(0.05, 2.0, size=(2, *shape)).astype(np.float32)
+        s, o = tau.FieldSolver(k), OracleFieldSolver(k)
+    elif kind == "multiphase":
+        img = _labels(shape, 3, 5)
+        s, o = tau.MultiPhaseSolver(img, dict(D3)), OracleMultiPhaseSolver(img, dict(D3))
+    elif kind == "anisotropic":
+        img = _labels(shape, 2, 5)
+        s, o = (c(img, (1.0, 1.3, 2.0)) for c in (tau.AnisotropicSolver, OracleAnisotropicSolver))
+    else:
+        img = _labels(shape, 3, 5)
+        cls, ocls = ((tau.ElectrodeSolver, OracleElectrodeSolver) if kind == "electrode" else
+                     (tau.PeriodicElectrodeSolver, OraclePeriodicElectrodeSolver))
+        s, o = cls(img), ocls(img)
+    assert s._resident_sweep()
+    s._resident.spin = 1
+    s.solve(iter_limit=130, verbose=False, conv_crit=0.0)
+    assert s._resident is False, "no wait ran out"
+    assert np.array_equal(s.field.cpu().numpy(), o.run(130).field.numpy())
